@@ -50,15 +50,19 @@ enum { VFD_PAD_CONSTANT_VF = 3, VFD_PAD_ZERO = 100 };
  *  VFD_KSPEC_SEPARABLE   a separable even kernel as FP64 tables
  *                        [scale | gx[px/2+1] | gy[py] | gz[pz] | R | g_0..g_16],
  *                        gz being the DFT of the normalized z window g of radius
- *                        R.  FP64 plans (and FP32 windows with R > 16): the z
- *                        pass forms K^(kz,ky,kx) = ((gx*gy)*scale)*gz in FP64
- *                        and rounds it to the plan's precision, the same numbers
- *                        VFD_KSPEC_REAL stores for the Gaussian.  FP32 plans with
- *                        R <= 16: the z pass convolves each z column with g
- *                        directly (the same operator; agrees with the FFT form to
- *                        FP32 rounding).  The form is chosen on the device from
- *                        the R stored in the table, so a table copied or moved
- *                        by any means runs the form its own R selects.
+ *                        R.  FP64 plans: the z pass forms K^(kz,ky,kx) =
+ *                        ((gx*gy)*scale)*gz in FP64, the same numbers
+ *                        VFD_KSPEC_REAL stores for the Gaussian.  FP32 plans:
+ *                        where gx, gy and gz are the DFTs of even windows of
+ *                        radius <= 31 that fit the zero padding, the tick is
+ *                        their direct convolution with the data (two passes, no
+ *                        transforms); otherwise the FFT passes, whose z pass
+ *                        convolves each z column with g directly for R <= 16 and
+ *                        multiplies by K^ rounded to FP32 beyond.  All forms are
+ *                        the same operator to FP32 rounding.  The form is found
+ *                        on the device from the tables of the call, on every
+ *                        call, so a table copied, moved or edited by any means
+ *                        runs the form its own contents select.
  *                        VFD_PAD_ZERO plans only. */
 enum { VFD_KSPEC_REAL = 0, VFD_KSPEC_COMPLEX_STD = 1, VFD_KSPEC_SEPARABLE = 2 };
 
@@ -123,13 +127,16 @@ int vfd_diffuse(const vfd_plan* plan, const vfd_field* fields, int nfields, void
 /* The five passes of vfd_diffuse, one at a time (same arguments), in order
  * VFD_PASS_XFWD, VFD_PASS_YFWD, VFD_PASS_ZCONV, VFD_PASS_YINV, VFD_PASS_XINV;
  * for per-pass timing.  In the XLAST order the same five indices run z R2C,
- * y forward, the fused x pass, y inverse and z C2R.  vfd_plan_pass_bytes gives the algorithmic HBM bytes
+ * y forward, the fused x pass, y inverse and z C2R.  A separable FP32 field of
+ * the direct form is done by the first pass (x and y windows, into work) and the
+ * last (z window); the passes between leave it alone.  vfd_plan_pass_bytes gives the algorithmic HBM bytes
  * of one pass for one field (sum over passes = bytes_per_field_tick). */
 enum { VFD_PASS_XFWD = 0, VFD_PASS_YFWD = 1, VFD_PASS_ZCONV = 2, VFD_PASS_YINV = 3, VFD_PASS_XINV = 4 };
-/* The single launches of the z pass, for per-kernel timing: the direct form
- * of radius bound 8, 12 and 16 (FP32 separable plans; no launch otherwise) and
- * the FFT form.  Each covers every field and acts on the fields of its own
- * form, so issuing all four equals VFD_PASS_ZCONV.  vfd_plan_pass_bytes gives
+/* Parts of the z pass, for per-kernel timing: the direct z pass for radius
+ * bound 8, 12 and 16 (FP32 separable plans; no launch otherwise; VFD_PASS_ZCONV
+ * has the three in one launch) and the FFT form.  Each covers every field and
+ * acts on the fields of its own form, so issuing all four equals
+ * VFD_PASS_ZCONV.  vfd_plan_pass_bytes gives
  * the bytes of one field of that form. */
 enum { VFD_PASS_Z_DIRECT8 = 5, VFD_PASS_Z_DIRECT12 = 6, VFD_PASS_Z_DIRECT16 = 7, VFD_PASS_Z_FFT = 8 };
 int vfd_diffuse_pass(const vfd_plan* plan, const vfd_field* fields, int nfields, int pass, void* stream);

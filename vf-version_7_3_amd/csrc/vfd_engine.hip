@@ -61,12 +61,16 @@ struct Shape {
     std::vector<void*> pool;  // work buffers of plan.work_bytes
     std::vector<char> held;   // 1 while a batch or a cached graph owns the buffer
     int nruns = 0;
+    bool fft_seen = false;    // a run with a field of the FFT form was admitted
 };
 
 struct Run {
     ShapeKey key{};
     int nfields = 0;
     std::vector<void*> field, kspec;
+    // window radius of the fields of the direct form (FP32), whose kspec array
+    // holds the form's record; -1: the FFT form, kspec holds the tables
+    std::vector<int> radius;
     size_t bytes = 0;
     bool busy = false;  // in an in-flight serving batch
 };
@@ -112,9 +116,14 @@ struct Branches {
     }
 };
 
-// the fields of one batch grouped by shape, with the work buffers they own
+// the fields of one batch grouped by shape and form, with the work buffers they own
+struct Group {
+    Shape* shape = nullptr;
+    int max_radius = -1;  // direct form: largest radius of the fields; -1: FFT form
+    std::vector<vfd_field> fields;
+};
 struct Batch {
-    std::vector<std::pair<Shape*, std::vector<vfd_field>>> groups;
+    std::vector<Group> groups;
     std::vector<Held> held;
 };
 
@@ -216,32 +225,37 @@ bool trim_pools(vfd_engine* e) {
     return any;
 }
 
-// Group the listed runs' fields by shape and reserve their work buffers
+// Group the listed runs' fields by shape and form and reserve their work buffers
 // (every allocation happens here, never while a stream is being captured).
 int build_batch(vfd_engine* e, const std::vector<int>& run_ids, Batch* bt) {
-    std::map<ShapeKey, std::vector<vfd_field>> groups;
+    std::map<std::pair<ShapeKey, bool>, Group> groups;
     for (int id : run_ids) {
         auto it = e->runs.find(id);
         if (it == e->runs.end()) return set_error(VFD_ERR_NOTFOUND, "step: unknown run %d", id);
         Run& r = it->second;
-        auto& g = groups[r.key];
-        for (int f = 0; f < r.nfields; ++f) g.push_back(vfd_field{r.field[f], r.field[f], nullptr, r.kspec[f], 0.0, 0, 0});
+        for (int f = 0; f < r.nfields; ++f) {
+            Group& g = groups[{r.key, r.radius[f] >= 0}];
+            g.max_radius = std::max(g.max_radius, r.radius[f]);
+            g.fields.push_back(vfd_field{r.field[f], r.field[f], nullptr, r.kspec[f], 0.0, 0, 0});
+        }
     }
     for (auto& kv : groups) {
-        Shape& s = e->shapes[kv.first];
+        const ShapeKey& key = kv.first.first;
+        Shape& s = e->shapes[key];
         Held h;
         const int by_bytes = (int)std::max<size_t>(1, group_work_bytes() / s.plan.work_bytes);
-        const int want = std::min({(int)kv.second.size(), kMaxFieldsPerLaunch, by_bytes});
+        const int want = std::min({(int)kv.second.fields.size(), kMaxFieldsPerLaunch, by_bytes});
         if (acquire(e, s, want, &h) < 1) {
             release(h);
             for (auto& hh : bt->held) release(hh);
             bt->held.clear();
             bt->groups.clear();
-            return set_error(VFD_ERR_BUDGET, "step: no work buffer fits the HBM budget for %dx%dx%d", kv.first.nx,
-                             kv.first.ny, kv.first.nz);
+            return set_error(VFD_ERR_BUDGET, "step: no work buffer fits the HBM budget for %dx%dx%d", key.nx, key.ny,
+                             key.nz);
         }
         bt->held.push_back(h);
-        bt->groups.emplace_back(&s, std::move(kv.second));
+        kv.second.shape = &s;
+        bt->groups.push_back(std::move(kv.second));
     }
     return VFD_OK;
 }
@@ -263,10 +277,17 @@ int launch_batch(Batch& bt, int ticks, hipStream_t st, Branches& br) {
         if (int rc = hip_check(hipEventRecord(br.fork, st), "fork")) return rc;
     }
     for (int gi = 0; gi < ng; ++gi) {
-        Shape& s = *bt.groups[gi].first;
-        std::vector<vfd_field>& fl = bt.groups[gi].second;
+        Group& g = bt.groups[gi];
+        Shape& s = *g.shape;
+        std::vector<vfd_field>& fl = g.fields;
         const Held& h = bt.held[gi];
-        const size_t k = h.idx.size();
+        // the direct form keeps one real field between its passes: a work buffer
+        // (the FFT form's padded half spectrum) has room for several
+        const bool direct = g.max_radius >= 0;
+        const size_t slot = (s.plan.field_bytes + 255) / 256 * 256;
+        const size_t per_buf = direct ? std::max<size_t>(1, s.plan.work_bytes / slot) : 1;
+        size_t k = h.idx.size() * per_buf;
+        if (direct) k = std::min<size_t>({k, (size_t)kMaxFieldsPerLaunch, std::max<size_t>(1, group_work_bytes() / slot)});
         hipStream_t gs = fork ? br.aux[gi % kAuxStreams] : st;
         if (fork) {
             if (int rc = hip_check(hipStreamWaitEvent(gs, br.fork, 0), "fork wait")) return rc;
@@ -274,8 +295,12 @@ int launch_batch(Batch& bt, int ticks, hipStream_t st, Branches& br) {
         for (int t = 0; t < ticks; ++t)
             for (size_t c = 0; c < fl.size(); c += k) {
                 const int n = (int)std::min(k, fl.size() - c);
-                for (int i = 0; i < n; ++i) fl[c + i].work = s.pool[h.idx[i]];
-                if (int rc = plan_diffuse(s.plan, fl.data() + c, n, gs)) return rc;
+                // spread over the buffers first, then over the slots of each
+                for (int i = 0; i < n; ++i)
+                    fl[c + i].work = (char*)s.pool[h.idx[i % h.idx.size()]] + i / h.idx.size() * slot;
+                const int rc = direct ? plan_diffuse_direct(s.plan, fl.data() + c, n, g.max_radius, 0, 5, gs)
+                                      : plan_diffuse(s.plan, fl.data() + c, n, gs, Form::fft);
+                if (rc) return rc;
             }
         if (fork) {
             if (int rc = hip_check(hipEventRecord(br.join[gi % kAuxStreams], gs), "join")) return rc;
@@ -511,23 +536,36 @@ static int run_create(vfd_engine* e, const vfd_run_desc* d, int* run_id, double 
         }
         if (!rc) {
             r.kspec.push_back(kp);
-            rc = hip_check(hipMemset(fp, 0, plan.field_bytes), "run field clear");
+            r.radius.push_back(-1);
+            rc = plan_gauss_spectrum(plan, d->sigma2[f], d->decay[f], kp, nullptr);
         }
-        if (!rc) rc = plan_gauss_spectrum(plan, d->sigma2[f], d->decay[f], kp, nullptr);
+        // the field's form, decided from its table once: nobody else writes it.
+        // The record takes the table's place (made in the field's own memory,
+        // which is cleared next); smaller arrays keep the FFT form.
+        if (!rc && plan.direct && std::min(plan.field_bytes, plan.kspec_bytes) >= kDirRecordBytes) {
+            rc = plan_direct_record(plan, kp, fp, &r.radius[f], nullptr);
+            if (!rc && r.radius[f] >= 0)
+                rc = hip_check(hipMemcpyAsync(kp, fp, kDirRecordBytes, hipMemcpyDeviceToDevice, nullptr), "run record");
+        }
+        if (!rc) rc = hip_check(hipMemset(fp, 0, plan.field_bytes), "run field clear");
     }
     std::vector<void*> frees;
     size_t unreserve = 0;
     {
         std::lock_guard<std::mutex> lk(e->mu);
         Shape& s = e->shapes.find(key)->second;  // kept by the nruns count taken above
-        if (reserved_work) {
-            // schedule for a new shape, tuned once per process on scratch buffers
-            // when they fit (plan_init took a cached schedule: a shape whose runs
-            // all left and that comes back is not tuned again)
+        // schedule of the FFT passes for the shape's first run that needs them,
+        // tuned once per process on scratch buffers when they fit (plan_init took
+        // a cached schedule: a shape whose runs all left and that comes back is
+        // not tuned again)
+        if (!rc && !s.fft_seen && std::find(r.radius.begin(), r.radius.end(), -1) != r.radius.end()) {
+            s.fft_seen = true;
             const int nf = std::min(8, d->nfields);
-            if (!rc && !getenv("VFD_NO_AUTOTUNE") && !tuned_known(s.plan) &&
+            if (!getenv("VFD_NO_AUTOTUNE") && !tuned_known(s.plan) &&
                 e->used + (size_t)nf * (plan.work_bytes + plan.field_bytes + plan.kspec_bytes) <= e->budget)
                 (void)plan_autotune(s.plan, nf, nullptr, nullptr);
+        }
+        if (reserved_work) {
             e->used -= reserved_work;  // the shape's first work buffer is charged by acquire
             reserved -= reserved_work;
             Held h;
@@ -679,7 +717,9 @@ int vfd_step_plain(vfd_engine* e, const int* run_ids, int nruns, int ticks, void
             for (int f = 0; f < r.nfields; ++f) {
                 vfd_field fl{r.field[f], r.field[f], s.pool[h.idx[0]], r.kspec[f], 0.0, 0, 0};
                 for (int pass = 0; pass < 5; ++pass)
-                    if (int rc = plan_diffuse_passes(s.plan, &fl, 1, pass, pass + 1, st)) {
+                    if (int rc = r.radius[f] >= 0
+                                     ? plan_diffuse_direct(s.plan, &fl, 1, r.radius[f], pass, pass + 1, st)
+                                     : plan_diffuse_passes(s.plan, &fl, 1, pass, pass + 1, st, nullptr, Form::fft)) {
                         release(h);
                         return rc;
                     }

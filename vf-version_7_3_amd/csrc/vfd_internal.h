@@ -28,7 +28,17 @@ struct Plan {
     int hz;        // x-last: pz/2 + 1 z half-spectrum planes
     long ldx;      // x-last: work row stride (complex elements)
     long xplane;   // x-last: work plane stride py * ldx
+    // FP32 separable plans: a tick may take the direct convolution; the record
+    // of a call's field sits at this offset of its work array (the last bytes)
+    bool direct;
+    size_t rec_off;
 };
+
+// Which form the fields of a call take (FP32 separable plans).
+//  by_table: decided on the device from each field's table, on every call;
+//  direct:   known to have the direct form, kspec is the field's DirRecord;
+//  fft:      the FFT passes.
+enum class Form { by_table, direct, fft };
 
 int set_error(int code, const char* fmt, ...);
 int hip_check(hipError_t e, const char* what);
@@ -38,7 +48,14 @@ int plan_init(const vfd_plan_desc* d, Plan* p);
 void tuned_lookup(Plan& q);
 bool tuned_known(const Plan& q);  // a tuned schedule of this shape is cached
 int plan_autotune(Plan& p, int nfields, hipStream_t st, float* best_ms);
-int plan_diffuse(const Plan& p, const vfd_field* fields, int nfields, hipStream_t st);
+int plan_diffuse(const Plan& p, const vfd_field* fields, int nfields, hipStream_t st, Form form = Form::by_table);
+// Form::direct: largest window radius among the fields
+int plan_diffuse_direct(const Plan& p, const vfd_field* fields, int nfields, int max_radius, int lo, int hi,
+                        hipStream_t st);
+// The DirRecord of a table into `rec` (device, kDirRecordBytes, outside the
+// table), and from there to the host; *radius = the largest of the three window
+// radii, or -1 when the table has no direct form.  Synchronizes.
+int plan_direct_record(const Plan& p, const void* d_kspec, void* rec, int* radius, hipStream_t st);
 float chem_display_scale(int chem);  // sampleChem's per-chem display scale, chem < 8
 int chem_levels(float* d_p, const float* d_t, float* d_d, float decay, long n, hipStream_t st);
 int chem_grads_totals(float* const* d_p, const float* d_frag_col, const float* d_frag_ela, float* const* d_grads,
@@ -55,7 +72,7 @@ struct Epilogue {
     int vis_stride = 0;
 };
 int plan_diffuse_passes(const Plan& p, const vfd_field* fields, int nfields, int lo, int hi, hipStream_t st,
-                        const Epilogue* epi = nullptr);
+                        const Epilogue* epi = nullptr, Form form = Form::by_table);
 double plan_pass_bytes(const Plan& p, int pass);
 int plan_gauss_spectrum(const Plan& p, double sigma2, double decay, void* d_kspec, hipStream_t st);
 int plan_mass(const Plan& p, const void* const* d_fields, int nfields, double* mass, hipStream_t st);

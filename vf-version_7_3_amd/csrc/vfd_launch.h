@@ -27,10 +27,19 @@ template <typename T>
 hipError_t launch_col(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
                       const void* tw, hipStream_t st, int variant = 0);
 
-// direct z pass (FP32, separable spectrum) for window radius R <= rm, rm one of
-// 8, 12, 16 (kZDirectMaxR); cd.scale carries Pz.
-hipError_t launch_zdirect(int rm, const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
+// direct z pass of the FFT form (FP32, separable spectrum) for the fields whose
+// z window's radius class (8, 12, 16 = kZDirectMaxR) is in `classes` (bits 0, 1,
+// 2); cd.scale carries Pz.
+hipError_t launch_zdirect(unsigned classes, const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
                           hipStream_t st);
+
+// Direct-convolution form (vfd_direct.hpp), FP32 separable fields: the records
+// of the batch, the x-y pass (in -> work) and the z pass (work -> out).  Both
+// passes act on the fields whose record has the form; max_radius bounds their
+// radii (the launch's LDS), kDirMaxR where the host does not know them.
+hipError_t launch_dir_classify(const FieldBatch& fields, int nfields, const DirDims& d, hipStream_t st);
+hipError_t launch_dir_xy(const FieldBatch& fields, int nfields, const DirDims& d, hipStream_t st);
+hipError_t launch_dir_z(const FieldBatch& fields, int nfields, const DirDims& d, hipStream_t st, bool vis);
 
 // x-last order (FP32): z R2C (fwd) / C2R (inverse) of column pairs with FFT
 // length pz, and the fused x row pass of length px.  xlast_supported tells

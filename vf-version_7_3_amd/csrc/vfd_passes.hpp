@@ -90,6 +90,21 @@ template <typename T> struct RowLds {
     __device__ __forceinline__ cx<T>& at(int n) { return base[n + (n >> 5)]; }
 };
 
+// Whether a field's tick goes through the direct convolution (vfd_direct.hpp):
+// the launches of the FFT passes then leave it alone.
+__device__ __forceinline__ bool dir_skip(const FieldDesc& fd) {
+    if (!fd.dir) return false;
+    const DirRecord* r = (const DirRecord*)fd.dir;
+    return r->ax[0].radius >= 0 && r->ax[1].radius >= 0 && r->ax[2].radius >= 0;
+}
+
+// The last item of `item`'s field in a work-group's sequence item, item + step,
+// ... (ngroups items per field): where its loop continues after a skipped field.
+__device__ __forceinline__ long field_end(long item, long ngroups, long step) {
+    const long left = (item / ngroups + 1) * ngroups - 1 - item;
+    return item + left / step * step;
+}
+
 // ------------------------------------------------------------- x forward
 // rows r = z*Ny + y (z < Nz, y < Ny).  Packed z[n] = u(2n) + i u(2n+1) of the
 // padded row (length L = Px/2), length-L FFT, then the real-FFT post-process
@@ -121,6 +136,12 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
         const int f = (int)(item / ngroups);
         const long row = (item % ngroups) * C::G + gr;
         const FieldDesc& fd = fb.f[f];
+        if constexpr (sizeof(T) == 4) {
+            if (dir_skip(fd)) {  // work-group uniform: on to the next field's groups
+                item = field_end(item, ngroups, gridDim.x);
+                continue;
+            }
+        }
         const auto rin = B::make(fd.in, g.in_bytes);
         const auto rwork = B::make(fd.work, g.work_bytes);
         const bool live = row < nrows;
@@ -218,6 +239,12 @@ xinv_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
         const int f = (int)(item / ngroups);
         const long row = (item % ngroups) * C::G + gr;
         const FieldDesc& fd = fb.f[f];
+        if constexpr (sizeof(T) == 4) {
+            if (dir_skip(fd)) {
+                item = field_end(item, ngroups, gridDim.x);
+                continue;
+            }
+        }
         const auto rwork = B::make(fd.work, g.work_bytes);
         const auto rout = B::make(fd.out, g.out_bytes);
         const bool live = row < nrows;
@@ -435,6 +462,9 @@ col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
         if (bz >= cd.grid_fields || (long)bx * C::TC >= cd.ncols) return;
     }
     const FieldDesc& fd = fb.f[bz];
+    if constexpr (sizeof(T) == 4) {
+        if (dir_skip(fd)) return;  // whole-block exit
+    }
     if constexpr (SEP && sizeof(T) == 4) {
         // FP32 separable tables of radius <= kZDirectMaxR take the direct z pass
         // (zdirect_kernel, launched over the same fields); whole-block exit
@@ -659,21 +689,18 @@ col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
 // lane streams its column once: the window of 2 RM + 1 values lives in
 // registers, rotated at compile time inside blocks of U = 2 RM + 1 outputs,
 // and row n + RM is loaded before row n is written, so the pass is in place.
-// RM is a compile-time bound on R; the table holds zero taps beyond R.  A
-// launch covers every field of the batch: a work-group whose table's radius
-// is not in this RM's range (zform_of) exits at once.
+// RM is a compile-time bound on R; the table holds zero taps beyond R.  The
+// launch covers every field of the batch: a work-group whose table's radius is
+// in no class of the launch (zform_of) exits at once.
 
 template <int RM>
-__global__ void __launch_bounds__(64)
-zdirect_kernel(const FieldBatch fb, ColDesc cd) {
+__device__ __forceinline__ void zdirect_column(const FieldDesc& fd, const ColDesc& cd) {
     using B = BufOps<float>;
     using O = typename B::O;
     using BD = BufOps<double>;
     using OD = typename BD::O;
     constexpr int U = 2 * RM + 1;
     constexpr unsigned CB = sizeof(cx<float>);
-    const FieldDesc& fd = fb.f[blockIdx.z];
-    if (zform_of_table(fd.kspec, cd.kspec_bytes, cd.sep_g) != RM) return;
     const auto rwork = B::make(fd.work, cd.work_bytes);
     const long col = (long)blockIdx.x * 64 + threadIdx.x;
     const long ky = blockIdx.y;

@@ -231,6 +231,13 @@ int plan_init(const vfd_plan_desc* d, Plan* p) {
         return set_error(VFD_ERR_UNSUPPORTED,
                          "plan: a per-field FP32 array exceeds 4 GiB (work %zu, spectrum %zu, field %zu bytes)",
                          q.work_bytes, q.kspec_bytes, q.field_bytes);
+    // the direct-convolution form (vfd_direct.hpp): its record follows the FFT
+    // passes' work array, whose front holds the pass between x-y and z
+    q.direct = q.prec == VFD_F32 && q.kspec_format == VFD_KSPEC_SEPARABLE;
+    if (q.direct) {
+        q.rec_off = round_up((long)std::max(q.work_bytes, q.field_bytes), 256);
+        q.work_bytes = q.rec_off + kDirRecordBytes;
+    }
     // pruned 5-pass algorithmic bytes: 8N + 32 A1 + 32 A2 + 4 A3 (FP32); the
     // complex terms scale with the precision and K^ with its element size.
     const double N = (double)q.nx * q.ny * q.nz;
@@ -280,25 +287,23 @@ int plan_init(const vfd_plan_desc* d, Plan* p) {
     return VFD_OK;
 }
 
-// z pass.  FP32 fields with a separable table take the direct form when the
-// table's window radius R is at most kZDirectMaxR, else the FFT form.  The
-// form is decided on the device from the R the table stores: the direct
-// launches (radius bounds 8, 12, 16) and the FFT launch each cover every field
-// of the batch, and a work-group whose field is not of its form exits at once
-// (zform_of in vfd_passes.hpp), so no host-side record of the tables is needed.
+// z pass of the FFT form.  FP32 fields with a separable table take the direct z
+// pass when the table's z window radius R is at most kZDirectMaxR, else the FFT
+// one.  That is decided on the device from the R the table stores: the direct
+// launch and the FFT launch each cover every field of the batch, and a
+// work-group whose field is not of its form exits at once (zform_of in
+// vfd_passes.hpp), so no host-side record of the tables is needed.
 // part selects one launch (0, 1, 2: the direct form of radius bound 8, 12,
 // 16; 3: the FFT form) for per-kernel timing, -1 all of them.
 template <typename T>
 static hipError_t launch_z(const Plan& p, const FieldBatch& fb, int nf, const ColDesc& z, hipStream_t st,
                            int part = -1) {
     if constexpr (sizeof(T) == 4) {
-        if (p.kspec_format == VFD_KSPEC_SEPARABLE) {
+        if (p.kspec_format == VFD_KSPEC_SEPARABLE && part != 3) {
             ColDesc zd = z;
             zd.scale = (double)p.pz;
-            const int rms[3] = {8, 12, 16};
-            for (int i = 0; i < 3; ++i)
-                if (part < 0 || part == i)
-                    if (hipError_t e = launch_zdirect(rms[i], fb, nf, zd, p.py, st)) return e;
+            const unsigned classes = part < 0 ? 7u : 1u << part;
+            if (hipError_t e = launch_zdirect(classes, fb, nf, zd, p.py, st)) return e;
         }
     }
     if (part >= 0 && part != 3) return hipSuccess;
@@ -345,9 +350,20 @@ static int run_xlast(const Plan& p, const FieldBatch& fb, int nf, int pass_lo, i
     return VFD_OK;
 }
 
+static DirDims dir_dims(const Plan& p, int max_radius) {
+    DirDims d{};
+    d.nx = p.nx; d.ny = p.ny; d.nz = p.nz;
+    d.px = p.px; d.py = p.py; d.pz = p.pz;
+    d.max_radius = max_radius;
+    d.bytes = p.field_bytes;
+    return d;
+}
+
 template <typename T>
 static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pass_lo, int pass_hi,
-                    hipStream_t st, const Epilogue* epi, int zpart = -1) {
+                    hipStream_t st, const Epilogue* epi, int zpart = -1, Form form = Form::by_table,
+                    int max_radius = kDirMaxR) {
+    const bool records = p.direct && form != Form::fft;
     for (int f0 = 0; f0 < nfields; f0 += kMaxFieldsPerLaunch) {
         const int nf = std::min(kMaxFieldsPerLaunch, nfields - f0);
         FieldBatch fb;
@@ -360,6 +376,7 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
             fb.f[i].kspec = f.kspec;
             fb.f[i].base = f.base;
             fb.f[i].epi = f.epi;
+            if (records) fb.f[i].dir = form == Form::direct ? f.kspec : (char*)f.work + p.rec_off;
             if (epi && epi->deltas) {
                 fb.f[i].delta = epi->deltas[f0 + i];
                 fb.f[i].decay = epi->decay[f0 + i];
@@ -370,13 +387,14 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
                 fb.f[i].vis_stride = epi->vis_stride;
             }
         }
+        const size_t work_bytes = p.direct ? p.rec_off : p.work_bytes;  // without the record
         GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, p.pad_mode, p.kspec_format == VFD_KSPEC_COMPLEX_STD,
-                   p.field_bytes, p.work_bytes, p.kspec_bytes, p.field_bytes,
+                   p.field_bytes, work_bytes, p.kspec_bytes, p.field_bytes,
                    p.kspec_format == VFD_KSPEC_COMPLEX_STD ? 1.0 : (double)p.px * p.py * p.pz};
         ColDesc y{};
         y.mode = COL_FWD; y.rs = p.rs_y; y.nin = p.ny; y.nout = p.py; y.ncols = p.hx;
         y.rstride = p.ld; y.pstride = p.plane; y.scale = 1.0;
-        y.work_bytes = p.work_bytes; y.kspec_bytes = p.kspec_bytes;
+        y.work_bytes = work_bytes; y.kspec_bytes = p.kspec_bytes;
         ColDesc z{};
         z.mode = COL_FUSED; z.rs = p.rs_z; z.nin = p.nz; z.nout = p.nz; z.ncols = p.hx;
         z.rstride = p.plane; z.pstride = p.ld; z.ks_row = p.ks_row; z.ks_plane = p.ks_plane;
@@ -387,7 +405,7 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
         z.sep_g = 1 + p.hx + p.py + p.pz;
         // the real native spectrum carries the 1/(px py pz) normalization
         z.scale = z.kspec_complex ? 1.0 / ((double)p.px * p.py * p.pz) : 1.0;
-        z.work_bytes = p.work_bytes; z.kspec_bytes = p.kspec_bytes;
+        z.work_bytes = work_bytes; z.kspec_bytes = p.kspec_bytes;
         ColDesc yi = y;
         yi.mode = COL_INV; yi.nin = p.py; yi.nout = p.ny;
         if (p.fold_y) { yi.rs = 2; yi.fold = 1; }
@@ -398,8 +416,20 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
                 continue;
             }
         }
+        // The direct form's x-y pass goes with the first pass of the FFT form and
+        // its z pass with the last: in between it is the FFT fields' work alone.
+        const DirDims dd = dir_dims(p, max_radius);
         for (int pass = pass_lo; pass < pass_hi; ++pass) {
             hipError_t e = hipSuccess;
+            if constexpr (sizeof(T) == 4) {
+                if (records) {
+                    if (pass == VFD_PASS_XFWD && form == Form::by_table) e = launch_dir_classify(fb, nf, dd, st);
+                    if (pass == VFD_PASS_XFWD && e == hipSuccess) e = launch_dir_xy(fb, nf, dd, st);
+                    if (pass == VFD_PASS_XINV) e = launch_dir_z(fb, nf, dd, st, epi && epi->vis);
+                    if (e != hipSuccess) return hip_check(e, "direct pass launch");
+                    if (form == Form::direct) continue;
+                }
+            }
             switch (pass) {
                 case VFD_PASS_XFWD: e = launch_xfwd<T>(p.L, fb, nf, g, p.tw_x, st, p.var[pass]); break;
                 case VFD_PASS_YFWD: e = launch_col<T>(p.qy, fb, nf, y, p.nz, p.tw_y, st, p.var[pass]); break;
@@ -424,12 +454,35 @@ static int check_fields(const vfd_field* fields, int nfields) {
 }
 
 int plan_diffuse_passes(const Plan& p, const vfd_field* fields, int nfields, int lo, int hi, hipStream_t st,
-                        const Epilogue* epi) {
+                        const Epilogue* epi, Form form) {
     if (int rc = check_fields(fields, nfields)) return rc;
     if (lo < 0 || hi > 5 || lo >= hi) return set_error(VFD_ERR_INVALID, "diffuse: bad pass range [%d,%d)", lo, hi);
     if (nfields == 0) return VFD_OK;
-    return p.prec == VFD_F32 ? run_tick<float>(p, fields, nfields, lo, hi, st, epi)
+    return p.prec == VFD_F32 ? run_tick<float>(p, fields, nfields, lo, hi, st, epi, -1, form)
                              : run_tick<double>(p, fields, nfields, lo, hi, st, epi);
+}
+
+int plan_diffuse_direct(const Plan& p, const vfd_field* fields, int nfields, int max_radius, int lo, int hi,
+                        hipStream_t st) {
+    if (int rc = check_fields(fields, nfields)) return rc;
+    if (!p.direct) return set_error(VFD_ERR_INVALID, "diffuse: plan has no direct form");
+    if (nfields == 0) return VFD_OK;
+    return run_tick<float>(p, fields, nfields, lo, hi, st, nullptr, -1, Form::direct, max_radius);
+}
+
+int plan_direct_record(const Plan& p, const void* d_kspec, void* rec, int* radius, hipStream_t st) {
+    FieldBatch fb;
+    memset(&fb, 0, sizeof fb);
+    fb.f[0].kspec = d_kspec;
+    fb.f[0].dir = rec;
+    if (int rc = hip_check(launch_dir_classify(fb, 1, dir_dims(p, kDirMaxR), st), "classify launch")) return rc;
+    DirRecord h;
+    if (int rc = hip_check(hipMemcpyAsync(&h, rec, sizeof h, hipMemcpyDeviceToHost, st), "record download")) return rc;
+    if (int rc = hip_check(hipStreamSynchronize(st), "record sync")) return rc;
+    *radius = std::max({h.ax[0].radius, h.ax[1].radius, h.ax[2].radius});
+    for (const DirAxis& a : h.ax)
+        if (a.radius < 0) *radius = -1;
+    return VFD_OK;
 }
 
 // one launch of the z pass (part 0..3, see launch_z)
@@ -477,8 +530,8 @@ double plan_pass_bytes(const Plan& p, int pass) {
     }
 }
 
-int plan_diffuse(const Plan& p, const vfd_field* fields, int nfields, hipStream_t st) {
-    return plan_diffuse_passes(p, fields, nfields, 0, 5, st);
+int plan_diffuse(const Plan& p, const vfd_field* fields, int nfields, hipStream_t st, Form form) {
+    return plan_diffuse_passes(p, fields, nfields, 0, 5, st, nullptr, form);
 }
 
 // Fills scratch with hashed values in [0, 1) (as FP32 words): timings on
@@ -537,7 +590,7 @@ int plan_autotune(Plan& p, int nfields, hipStream_t st, float* best_ms) {
         int rc2 = VFD_OK;
         for (int q = 0; q < 5 && !rc2; ++q) {
             if (q == pass) rc2 = hip_check(hipEventRecord(e0, st), "event");
-            if (!rc2) rc2 = plan_diffuse_passes(p, fl.data(), nfields, q, q + 1, st);
+            if (!rc2) rc2 = plan_diffuse_passes(p, fl.data(), nfields, q, q + 1, st, nullptr, Form::fft);
             if (!rc2 && q == pass) rc2 = hip_check(hipEventRecord(e1, st), "event");
         }
         if (!rc2 && ms) rc2 = hip_check(hipEventSynchronize(e1), "event sync");

@@ -24,6 +24,9 @@ struct FieldDesc {
     float* vis;         //   min(t * vis_scale, 1) into a dense [Nz/s][Ny/s][Nx/s] array
     float vis_scale;
     int pad2_;
+    // FP32 separable fields: the field's DirRecord; a launch of the FFT passes
+    // skips a field whose record has the direct form (null: no record, FFT form)
+    const void* dir;
 };
 
 // Fields of one launch, passed by value as a kernel argument (graph-capture
@@ -87,6 +90,31 @@ struct XlDesc {
     unsigned long in_bytes, work_bytes, kspec_bytes, out_bytes;  // per-field array sizes
     // grouped 1-D launch of narrow tiles (set by the launcher)
     unsigned grid_fields, grid_segs;
+};
+
+// The direct-convolution form of one separable FP32 field (vfd_direct.hpp).
+// Windows up to kDirMaxR take it; its cost grows with 2 R + 1 per axis, and at
+// R = 31 it is still a fraction of the FFT passes' time.
+constexpr int kDirMaxR = 31;
+struct DirAxis {
+    double gain;               // exact window sum / sum of the FP32 taps (1 where not all taps are >= 0)
+    int radius;                // -1: the axis' table is not a short window
+    float tap[kDirMaxR + 1];   // h_0 .. h_R, then zeros
+};
+struct DirRecord {
+    double scale;              // table scale * px py pz
+    DirAxis ax[3];             // x, y, z
+};
+constexpr unsigned long kDirRecordBytes = 512;
+static_assert(sizeof(DirRecord) <= kDirRecordBytes, "record size");
+
+struct DirDims {
+    int nx, ny, nz, px, py, pz;
+    unsigned nfields;
+    unsigned xtiles, ychunks;  // dir_xy: strips per row, march chunks per plane
+    int yrows;                 // rows per chunk
+    int max_radius;            // largest radius the launch's LDS holds
+    unsigned long bytes;       // of one real field
 };
 
 // Largest window radius the direct z pass takes (separable spectrum, FP32);
