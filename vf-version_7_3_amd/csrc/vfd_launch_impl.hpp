@@ -18,6 +18,23 @@
 
 namespace vfd {
 
+// The schedule of the lengths and precisions compiled in one variant only:
+// radix 8, 8 elements per thread.  Against radix 16 it has half the registers
+// per thread and so about twice the waves, worth more than the saved stage:
+//  FP64 (a complex value takes 4 registers): z pass of 4 fields 256x128x64
+//   252 -> 157 us, y inverse 97 -> 76, x passes 51 + 60 -> 49 + 49; a tick of 8
+//   fields 130x100x40 394 -> 313 us, of 2 fields 512x256x128 1982 -> 1550 us;
+//  FP32 (rows with 512-thread, columns with 256-thread work-groups): ticks of
+//   301x187x75 (8 fields) 1418 -> 1165 us, 560x51x90 (6) 711 -> 497, 140x100x40
+//   (8) 187 -> 160, 1100x600x36 (2) 1992 -> 1713.
+// Columns of 144 keep radix 16 (16 9 in three stages against 8 2 3 3 in four,
+// with only 16 columns a work-group): fused z pass 660 against 802 us.
+#ifdef VFD_ROW_TU
+template <typename T, int Q> constexpr int single_var() { return 1; }
+#else
+template <typename T, int Q> constexpr int single_var() { return sizeof(T) == 4 && Q == 144 ? 0 : 2; }
+#endif
+
 // resident work-groups per CU for a kernel (callers cache it per instantiation)
 template <typename K>
 static int blocks_per_cu(K kernel, int nt) {
@@ -71,16 +88,16 @@ static hipError_t row_var(int variant, const FieldBatch& fields, int nfields, co
 template <bool FWD>
 static hipError_t row_dispatch(int L, int variant, const FieldBatch& fields, int nfields, const GridDesc& g,
                                const void* tw, hipStream_t st) {
-    constexpr bool kVariants = sizeof(VFD_REAL) == 4;  // FP64 keeps the default schedule
+    constexpr bool kVariants = sizeof(VFD_REAL) == 4;  // FP64 has one schedule
     switch (L) {
 #define VFD_HOT(Q)                                                                   \
     case Q:                                                                          \
         if constexpr (kVariants)                                                     \
             return row_var<VFD_REAL, Q, FWD>(variant, fields, nfields, g, tw, st);   \
         else                                                                         \
-            return row_go<VFD_REAL, Q, 0, FWD>(fields, nfields, g, tw, st);
+            return row_go<VFD_REAL, Q, single_var<VFD_REAL, Q>(), FWD>(fields, nfields, g, tw, st);
 #define VFD_COLD(Q) \
-    case Q: return row_go<VFD_REAL, Q, 0, FWD>(fields, nfields, g, tw, st);
+    case Q: return row_go<VFD_REAL, Q, single_var<VFD_REAL, Q>(), FWD>(fields, nfields, g, tw, st);
         VFD_HOT_LENGTHS(VFD_HOT)
         VFD_COLD_LENGTHS(VFD_COLD)
 #undef VFD_HOT
@@ -96,16 +113,20 @@ hipError_t launch_xfwd<VFD_REAL>(int L, const FieldBatch& fields, int nfields, c
     return row_dispatch<true>(L, variant, fields, nfields, g, tw, st);
 }
 
-// x inverse with the fused visualisation downsample: FP32, default schedule
+// x inverse with the fused visualisation downsample: FP32, the default schedule
+// of the length (the one vfd_diffuse runs untuned)
 static hipError_t xinv_vis(int L, const FieldBatch& fields, int nfields, const GridDesc& g, const void* tw,
                            hipStream_t st) {
     if constexpr (sizeof(VFD_REAL) == 4) {
         switch (L) {
-#define VFD_ANY(Q) \
+#define VFD_HOT(Q) \
     case Q: return row_go<VFD_REAL, Q, 0, false, true>(fields, nfields, g, tw, st);
-            VFD_HOT_LENGTHS(VFD_ANY)
-            VFD_COLD_LENGTHS(VFD_ANY)
-#undef VFD_ANY
+#define VFD_COLD(Q) \
+    case Q: return row_go<VFD_REAL, Q, single_var<VFD_REAL, Q>(), false, true>(fields, nfields, g, tw, st);
+            VFD_HOT_LENGTHS(VFD_HOT)
+            VFD_COLD_LENGTHS(VFD_COLD)
+#undef VFD_HOT
+#undef VFD_COLD
             default:
                 return hipErrorInvalidValue;
         }
@@ -191,16 +212,16 @@ static hipError_t col_var(int variant, const FieldBatch& fields, int nfields, co
 template <>
 hipError_t launch_col<VFD_REAL>(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd,
                                 long nplanes, const void* tw, hipStream_t st, int variant) {
-    constexpr bool kVariants = sizeof(VFD_REAL) == 4;  // FP64 keeps the default schedule
+    constexpr bool kVariants = sizeof(VFD_REAL) == 4;  // FP64 has one schedule
     switch (Q) {
 #define VFD_HOT(QQ)                                                                     \
     case QQ:                                                                            \
         if constexpr (kVariants)                                                        \
             return col_var<VFD_REAL, QQ>(variant, fields, nfields, cd, nplanes, tw, st); \
         else                                                                            \
-            return col_mode<VFD_REAL, QQ, 0>(fields, nfields, cd, nplanes, tw, st);
+            return col_mode<VFD_REAL, QQ, single_var<VFD_REAL, QQ>()>(fields, nfields, cd, nplanes, tw, st);
 #define VFD_COLD(QQ) \
-    case QQ: return col_mode<VFD_REAL, QQ, 0>(fields, nfields, cd, nplanes, tw, st);
+    case QQ: return col_mode<VFD_REAL, QQ, single_var<VFD_REAL, QQ>()>(fields, nfields, cd, nplanes, tw, st);
         VFD_HOT_LENGTHS(VFD_HOT)
         VFD_COLD_LENGTHS(VFD_COLD)
 #undef VFD_HOT
