@@ -153,7 +153,7 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
         const int xhi = cvf ? (fd.epi < g.Nx ? fd.epi : g.Nx) : g.Nx;
         const int xlo = cvf ? 1 : 0;
         const T base = cvf ? (T)fd.base : T(0);
-        const bool vec = !cvf && (g.Nx % 2 == 0);
+        const bool vec = g.Nx % 2 == 0;
 
         cx<T> v[Sh::E];
 #pragma unroll
@@ -164,8 +164,12 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
                 const int x0 = 2 * n, x1 = 2 * n + 1;
                 cx<T> val;
                 if (vec) {
+                    // the pair in one load; the constant pad's faces are cut afterwards
                     const bool ok = n >= 0 && row_in && x1 < g.Nx;
                     val = B::template ld_cx<kStream>(rin, ok ? rowoff + (O)x0 * RB : B::OOB);
+                    if (cvf)
+                        val = cx<T>{ok && x0 >= xlo && x0 < xhi ? val.x - base : T(0),
+                                    ok && x1 >= xlo && x1 < xhi ? val.y - base : T(0)};
                 } else {
                     const bool ok0 = n >= 0 && row_in && x0 >= xlo && x0 < xhi;
                     const bool ok1 = n >= 0 && row_in && x1 >= xlo && x1 < xhi;
@@ -462,9 +466,6 @@ col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
         if (bz >= cd.grid_fields || (long)bx * C::TC >= cd.ncols) return;
     }
     const FieldDesc& fd = fb.f[bz];
-    if constexpr (sizeof(T) == 4) {
-        if (dir_skip(fd)) return;  // whole-block exit
-    }
     if constexpr (SEP && sizeof(T) == 4) {
         // FP32 separable tables of radius <= kZDirectMaxR take the direct z pass
         // (zdirect_kernel, launched over the same fields); whole-block exit
@@ -477,6 +478,11 @@ col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
     const bool live = col < cd.ncols;
     const O base = (O)((long)by * cd.pstride + col) * CB;
     const O rstep = (O)cd.rstride * CB;
+    if constexpr (sizeof(T) == 4) {
+        // whole-block exit; here, so that the other arguments are in flight
+        // with the record pointer
+        if (dir_skip(fd)) return;
+    }
     ColLds<T, C::TC> lds{smem + c};
     // non-temporal loads only when a tile row spans whole 128-byte lines: a
     // narrower tile (long columns) shares each line with its neighbours, which

@@ -566,7 +566,8 @@ int plan_autotune(Plan& p, int nfields, hipStream_t st, float* best_ms) {
     std::vector<vfd_field> fl(nfields);
     for (int i = 0; i < nfields; ++i) {
         char* f = buf + (size_t)i * per_field;
-        fl[i] = vfd_field{f, f, f + fbytes + p.kspec_bytes, f + fbytes, 0.0, 0, 0};
+        // (the constant pad's interior is the whole row: with epi = 0 no data is read)
+        fl[i] = vfd_field{f, f, f + fbytes + p.kspec_bytes, f + fbytes, 0.0, p.nx, 0};
     }
     if (!rc && p.kspec_format == VFD_KSPEC_SEPARABLE) {
         // real separable tables, so that the z pass runs the form their radius

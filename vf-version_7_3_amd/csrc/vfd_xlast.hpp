@@ -95,8 +95,11 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                 const bool zin = n >= 0 && n < d.nz && (!cvf || (n > 0 && n < d.nz - 1));
                 const O off = dcol + (O)(zin ? n : 0) * dstep;
                 cx<T> val;
-                if (vec && !cvf) {
-                    val = B::template ld_cx<NTP>(rin, zin && in0 ? off : B::OOB);
+                if (vec) {
+                    // the pair in one load (both voxels are in the row); the
+                    // constant pad's faces are cut afterwards
+                    val = B::template ld_cx<NTP>(rin, zin && (in0 || in1) ? off : B::OOB);
+                    if (cvf) val = cx<T>{zin && in0 ? val.x - base : T(0), zin && in1 ? val.y - base : T(0)};
                 } else {
                     const T a0 = B::template ld_r<NTP>(rin, zin && in0 ? off : B::OOB);
                     const T a1 = B::template ld_r<NTP>(rin, zin && in1 ? off + RB : B::OOB);
