@@ -31,19 +31,21 @@ namespace vfd {
 // (the tables of vfd_gauss_spectrum are, to about 1e-15), the table is even,
 // and no tap wraps around the box (R <= P - n).  Everything else -- wider
 // windows, uneven or arbitrary tables, NaN -- gets radius -1.
-// FP64 throughout, cosines by rotation (error below 1e-13 over P/64 steps).
-// A latency chain in a tick's first launch: 1024 threads, so that the inverse
-// is 32 taps x 32 slices of the frequencies and the forward one frequency per
-// thread (4.8 us at P = 2048; with 256 threads holding all taps each and one
-// thread forming the record it took 15).
+// FP64 throughout.  A latency chain in a tick's first launch: the table and the
+// box's cosines are staged in LDS (one entry and one cospi per thread), then
+// 1024 threads are 32 taps x 32 slices of the frequencies in the inverse and a
+// frequency each forward.
 constexpr int kDirTaps = kDirMaxR + 1, kDirSlices = 32, kClassifyThreads = kDirTaps * kDirSlices;
 static_assert(kDirTaps == 32, "a record's taps are one half wave");
+constexpr int kDirHalfMax = 2304;  // P / 2 of the longest box: twice the longest compiled length
 
 __global__ void __launch_bounds__(kClassifyThreads)
 dir_classify_kernel(const FieldBatch fb, DirDims d) {
+    __shared__ double tl[kDirHalfMax + 1], ct[kDirHalfMax + 1];  // entries; cos(2 pi m / P)
     __shared__ double part[kDirSlices][kDirTaps];
     __shared__ double h[kDirTaps];
     __shared__ int bad_s;
+    constexpr int NK = (kDirHalfMax + kClassifyThreads) / kClassifyThreads;  // frequencies per thread
     const int ax = blockIdx.x;
     const FieldDesc& fd = fb.f[blockIdx.y];
     const double* tab = (const double*)fd.kspec;
@@ -54,18 +56,34 @@ dir_classify_kernel(const FieldBatch fb, DirDims d) {
     const int K = P / 2;  // frequencies 0 .. K
     const int J = min(kDirMaxR, (P - 1) / 2);
     const int tid = threadIdx.x, j = tid % kDirTaps, sl = tid / kDirTaps;
+    auto wrap = [&](int m) { return m >= P ? m - P : m; };
+    auto cosine = [&](int m) { return ct[m <= K ? m : P - m]; };  // 0 <= m < P
     if (tid == 0) bad_s = 0;
+    // the mirrored entries of an even table agree: their mean stands for both,
+    // their difference is checked below
+    double asym[NK];
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+        const int k = tid + i * kClassifyThreads;
+        asym[i] = 0.0;
+        if (k <= K) {
+            const double a = t[k], b = ax == 0 || k == 0 ? a : t[P - k];
+            tl[k] = 0.5 * (a + b);
+            ct[k] = cospi(2.0 * (double)k / (double)P);
+            asym[i] = fabs(a - b);
+        }
+    }
+    __syncthreads();
     {
         // slice sl holds the frequencies sl, sl + 32, ...
-        double c, s, cs, ss, acc = 0.0;
-        sincospi(2.0 * (double)(j * sl % P) / (double)P, &s, &c);
-        sincospi(2.0 * (double)(j * kDirSlices % P) / (double)P, &ss, &cs);
+        int m = j * sl % P;
+        const int step = j * kDirSlices % P;
+        double acc = 0.0;
+#pragma unroll 4
         for (int k = sl; k <= K; k += kDirSlices) {
-            const double w = (k == 0 || 2 * k == P) ? t[k] : ax == 0 ? 2.0 * t[k] : t[k] + t[P - k];
-            acc = fma(w, c, acc);
-            const double cn = c * cs - s * ss;
-            s = s * cs + c * ss;
-            c = cn;
+            const double w = (k == 0 || 2 * k == P) ? tl[k] : 2.0 * tl[k];
+            acc = fma(w, cosine(m), acc);
+            m = wrap(m + step);
         }
         part[sl][j] = acc;
     }
@@ -83,19 +101,19 @@ dir_classify_kernel(const FieldBatch fb, DirDims d) {
     for (int i = 0; i < kDirTaps; ++i) gmax += (i ? 2.0 : 1.0) * fabs(h[i]);
     const double tol = 1e-12 * gmax;
     bool bad = !(gmax <= 1e30);  // out of FP32's range, NaN
-    for (int k = tid; k <= K; k += kClassifyThreads) {
-        double c1, s1;
-        sincospi(2.0 * (double)k / (double)P, &s1, &c1);
-        double c = c1, s = s1, r = h[0];
 #pragma unroll
-        for (int i = 1; i < kDirTaps; ++i) {
-            r = fma(2.0 * h[i], c, r);
-            const double cn = c * c1 - s * s1;
-            s = s * c1 + c * s1;
-            c = cn;
+    for (int i = 0; i < NK; ++i) {
+        const int k = tid + i * kClassifyThreads;
+        if (k <= K) {
+            double r = h[0];
+            int m = k;
+#pragma unroll 8
+            for (int q = 1; q < kDirTaps; ++q) {
+                r = fma(2.0 * h[q], cosine(m), r);
+                m = wrap(m + k);
+            }
+            bad |= !(fabs(r - tl[k]) <= tol) || !(asym[i] <= tol);  // also NaN
         }
-        bad |= !(fabs(r - t[k]) <= tol);  // also NaN
-        if (ax != 0 && k > 0) bad |= !(fabs(r - t[P - k]) <= tol);
     }
     if (bad) bad_s = 1;
     __syncthreads();
@@ -160,6 +178,10 @@ struct DirSums {
         for (int v = 0; v < kDirOut; ++v) lo[v] = hi[v] = 0.0f;
     }
     __device__ __forceinline__ float operator[](int v) const { return lo[v] + hi[v]; }
+    __device__ __forceinline__ void pin() {
+#pragma unroll
+        for (int v = 0; v < kDirOut; ++v) asm volatile("" : "+v"(lo[v]), "+v"(hi[v]));
+    }
     // input element idx (0 .. 7 + 2 RB4) of the run that starts RB4 before the
     // first of the 8 outputs
     template <int RB> __device__ __forceinline__ void add(const DirTaps<RB>& tp, float in, int idx) {
@@ -178,17 +200,25 @@ struct DirSums {
 template <int TX, int RB>
 __device__ __forceinline__ void dir_ring_conv(DirSums& acc, const DirTaps<RB>& tp, const float* ring, int start,
                                               int col) {
-    constexpr int RB4 = dir_r4(RB), RS = dir_ring_rows(TX, RB);
-#pragma unroll
-    for (int blk = 0; blk < (kDirOut + 2 * RB4) / 8; ++blk) {
+    constexpr int RB4 = dir_r4(RB), RS = dir_ring_rows(TX, RB), NB = (kDirOut + 2 * RB4) / 8;
+    float in[2][8];
+    auto fetch = [&](int blk) {
         int row = start + 8 * blk;  // wave-uniform; rings are whole 8-row blocks
         row = row >= RS ? row - RS : row;
         const float* p = ring + row * TX + col;
-        float in[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) in[e] = p[e * TX];
+        for (int e = 0; e < 8; ++e) in[blk & 1][e] = p[e * TX];
+    };
+    fetch(0);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc.template add<RB>(tp, in[e], 8 * blk + e);
+    for (int blk = 0; blk < NB; ++blk) {
+        if (blk + 1 < NB) fetch(blk + 1);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc.template add<RB>(tp, in[blk & 1][e], 8 * blk + e);
+        // Sums formed here, reads one block ahead: left alone, the compiler forms
+        // one output after the other (sinking the sums to their stores), with
+        // the whole run's inputs live (122 VGPRs at radius 31 instead of 80).
+        acc.pin();
     }
 }
 
@@ -318,7 +348,7 @@ __global__ void __launch_bounds__(kDirThreads) dir_xy_kernel(const FieldBatch fb
 }
 
 // z window of TX columns of the flattened (y, x) plane from c0
-template <int TX, int RB, bool VIS>
+template <int TX, int RB, bool VIS, int POL>
 __device__ __forceinline__ void dir_z_strip(float* ring, const FieldDesc& fd, const DirRecord* rec, const DirDims& d,
                                             unsigned c0) {
     constexpr int RB4 = dir_r4(RB), B = dir_batch(TX), RS = dir_ring_rows(TX, RB);
@@ -342,7 +372,7 @@ __device__ __forceinline__ void dir_z_strip(float* ring, const FieldDesc& fd, co
         for (int i = 0; i < NLD; ++i) {
             const int z = zb + lr + i * LSTEP;
             const bool ok = z >= 0 && z < d.nz;
-            q[i] = dir_ld4<kCacheDefault>(rw, ok ? (unsigned)z * np + lcol : 0u, ok ? left : 0);
+            q[i] = dir_ld4<POL>(rw, ok ? (unsigned)z * np + lcol : 0u, ok ? left : 0);
         }
     };
     const int cc = tid % TX, rg = __builtin_amdgcn_readfirstlane(tid / TX);
@@ -378,9 +408,16 @@ __device__ __forceinline__ void dir_z_strip(float* ring, const FieldDesc& fd, co
         if (b >= M0 && zo < d.nz) {
             int start = pos + 8 * rg - 2 * RB4;
             start = start < 0 ? start + RS : start >= RS ? start - RS : start;
+            unsigned off = ((unsigned)zo * np + col) * 4u;
+            // the deltas are on their way while the window is summed
+            float dl[kDirOut];
+            if (upd) {
+#pragma unroll
+                for (int v = 0; v < kDirOut; ++v)
+                    dl[v] = BufOps<float>::ld_r<kStream>(rdel, live && zo + v < d.nz ? off + (unsigned)v * np * 4u : kBufOOB);
+            }
             DirSums acc;
             dir_ring_conv<TX, RB>(acc, tz, ring, start, cc);
-            unsigned off = ((unsigned)zo * np + col) * 4u;
 #pragma unroll
             for (int v = 0; v < kDirOut; ++v) {
                 const bool ok = live && zo + v < d.nz;
@@ -394,8 +431,7 @@ __device__ __forceinline__ void dir_z_strip(float* ring, const FieldDesc& fd, co
                     }
                 }
                 if (upd) {
-                    const float dl = BufOps<float>::ld_r<kStream>(rdel, ok ? off : kBufOOB);
-                    o = upd_level(dl, o, fd.decay);
+                    o = upd_level(dl[v], o, fd.decay);
                     BufOps<float>::st_r<kStream>(0.0f, rdel, ok ? off : kBufOOB);
                 }
                 BufOps<float>::st_r<kStream>(o, rout, ok ? off : kBufOOB);
@@ -409,7 +445,8 @@ __device__ __forceinline__ void dir_z_strip(float* ring, const FieldDesc& fd, co
     }
 }
 
-template <int TX, bool VIS>
+// POL: cache policy of the loads (see launch_dir_z)
+template <int TX, bool VIS, int POL>
 __global__ void __launch_bounds__(kDirThreads) dir_z_kernel(const FieldBatch fb, DirDims d) {
     extern __shared__ __align__(16) float dir_lds[];
     const FieldDesc& fd = fb.f[blockIdx.y];
@@ -418,7 +455,7 @@ __global__ void __launch_bounds__(kDirThreads) dir_z_kernel(const FieldBatch fb,
     const int R = __builtin_amdgcn_readfirstlane(rec->ax[2].radius);
     if (R > d.max_radius) return;
 #define VFD_GO(RB) \
-    if (R <= RB) return dir_z_strip<TX, RB, VIS>(dir_lds, fd, rec, d, blockIdx.x * (unsigned)TX);
+    if (R <= RB) return dir_z_strip<TX, RB, VIS, POL>(dir_lds, fd, rec, d, blockIdx.x * (unsigned)TX);
     VFD_DIR_RADII(VFD_GO)
 #undef VFD_GO
 }
