@@ -129,3 +129,27 @@ def test_tables_of_other_kernels(vfd, orc):
         print(f"case {name}: rel-L2 {rel:.3e}", flush=True)
         assert rel <= 1e-6, name     # FP32 transforms of this box: 1.3e-7 (test_separable_spectrum_matches_real)
         assert np.array_equal(a, e) == direct, name
+
+
+@pytest.mark.parametrize("shape,radii", [((40, 150, 330), (9, 36, 17, 33, 38)), ((48, 600, 70), (40, 6, 33)),
+                                         ((64, 96, 120), (32,) * 9 + (31,))])
+def test_mixed_batches_leave_the_fft_passes_their_fields(vfd, orc, shape, radii):
+    """Batches of both forms, through both launch shapes of the FFT passes: one
+    work-group per tile, and -- a plan that has itself made tables of the direct
+    form only -- persistent launches walking the tiles of the fields that are
+    theirs (more tiles than work-groups at the first two shapes; y columns long
+    enough for narrow tiles at the second).  Every field has the bits it has
+    alone, and both shapes match the oracle."""
+    print(f"case mixed shape={shape} radii={radii}", flush=True)
+    plan = vfd.Plan(shape, kspec_format=vfd.KSPEC_SEPARABLE)
+    few = vfd.Plan(shape, kspec_format=vfd.KSPEC_SEPARABLE)
+    few.gauss_spectrum(_s2(5), 0.97)
+    u = orc.synth_field(shape, 77, nsrc=4)
+    tables = [plan.gauss_spectrum(_s2(r), 0.97) for r in radii]
+    refs = {r: orc.direct_separable(u, _s2(r), 0.97) for r in set(radii)}
+    for p in (plan, few):
+        got = _tick(vfd, p, u, tables)
+        for r, t, g in zip(radii, tables, got):
+            (alone,) = _tick(vfd, p, u, [t])
+            assert np.array_equal(alone, g), r
+            assert float(np.linalg.norm(g - refs[r]) / np.linalg.norm(refs[r])) <= 1e-5, r

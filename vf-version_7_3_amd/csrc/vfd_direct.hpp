@@ -37,7 +37,6 @@ namespace vfd {
 // frequency each forward.
 constexpr int kDirTaps = kDirMaxR + 1, kDirSlices = 32, kClassifyThreads = kDirTaps * kDirSlices;
 static_assert(kDirTaps == 32, "a record's taps are one half wave");
-constexpr int kDirHalfMax = 2304;  // P / 2 of the longest box: twice the longest compiled length
 
 __global__ void __launch_bounds__(kClassifyThreads)
 dir_classify_kernel(const FieldBatch fb, DirDims d) {
@@ -336,7 +335,7 @@ __global__ void __launch_bounds__(kDirThreads) dir_xy_kernel(const FieldBatch fb
     if (f >= d.nfields) return;  // padding ids
     const FieldDesc& fd = fb.f[f];
     const DirRecord* rec = (const DirRecord*)fd.dir;
-    if (!dir_skip(fd)) return;  // not of this form: the FFT passes do it
+    if (!dir_form(fd.dir)) return;  // the FFT passes do it
     const int R = __builtin_amdgcn_readfirstlane(max(rec->ax[0].radius, rec->ax[1].radius));
     const rsrc_t rin = make_rsrc(fd.in, d.bytes), rw = make_rsrc(fd.work, d.bytes);
     const int x0 = (int)tile * TX, y0 = (int)ch * d.yrows, y1 = min(d.ny, y0 + d.yrows);
@@ -451,7 +450,7 @@ __global__ void __launch_bounds__(kDirThreads) dir_z_kernel(const FieldBatch fb,
     extern __shared__ __align__(16) float dir_lds[];
     const FieldDesc& fd = fb.f[blockIdx.y];
     const DirRecord* rec = (const DirRecord*)fd.dir;
-    if (!dir_skip(fd)) return;  // not of this form: the FFT passes do it
+    if (!dir_form(fd.dir)) return;  // the FFT passes do it
     const int R = __builtin_amdgcn_readfirstlane(rec->ax[2].radius);
     if (R > d.max_radius) return;
 #define VFD_GO(RB) \

@@ -32,6 +32,10 @@ struct Plan {
     // of a call's field sits at this offset of its work array (the last bytes)
     bool direct;
     size_t rec_off;
+    // which tables the plan's own vfd_gauss_spectrum has made: bit 0 within the
+    // direct form's radius, bit 1 beyond.  A hint for the launch shape of the FFT
+    // passes (Records), never for what they do; accessed atomically
+    mutable int tables;
 };
 
 // Which form the fields of a call take (FP32 separable plans).

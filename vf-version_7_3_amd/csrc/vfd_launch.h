@@ -27,6 +27,10 @@ template <typename T>
 hipError_t launch_col(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
                       const void* tw, hipStream_t st, int variant = 0);
 
+// the FP32 column pass of a batch with RECORDS_FEW: launch_col calls it
+hipError_t launch_col_rec(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
+                          const void* tw, hipStream_t st, int variant);
+
 // direct z pass of the FFT form (FP32, separable spectrum) for the fields whose
 // z window's radius class (8, 12, 16 = kZDirectMaxR) is in `classes` (bits 0, 1,
 // 2); cd.scale carries Pz.

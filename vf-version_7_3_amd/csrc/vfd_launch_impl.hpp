@@ -67,7 +67,7 @@ static hipError_t row_go(const FieldBatch& fields, int nfields, const GridDesc& 
     // (x passes 1.34 -> 1.31 ms at 1024x512x128, 8 fields), while a work-group
     // per row group restages the twiddle table for every 4 rows (1.65 ms)
     static const int per_cu = blocks_per_cu(kern, C::NT);  // this instantiation's
-    const long cap = 4L * num_cus() * per_cu;
+    const long cap = (g.records == RECORDS_FEW ? 1L : 4L) * num_cus() * per_cu;
     const unsigned grid = (unsigned)(items < cap ? items : cap);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(C::NT), 0, st, fields, g, (const cx<T>*)tw, nfields);
     return hipGetLastError();
@@ -143,36 +143,62 @@ hipError_t launch_xinv<VFD_REAL>(int L, const FieldBatch& fields, int nfields, c
 #endif
 
 #ifdef VFD_COL_TU
+// launch geometry of the 1-D column launches (col_coords); false: too many ids
+template <typename C>
+static bool col_ids(ColDesc& g, int nfields, long nplanes) {
+    g.grid_planes = (unsigned)nplanes;
+    g.grid_fields = (unsigned)nfields;
+    unsigned long ids;
+    if constexpr (C::SH > 1) {  // 8 segment groups per 8 * SH ids
+        g.grid_segs = (unsigned)((g.ncols + C::TC_LINE - 1) / C::TC_LINE);
+        ids = ((unsigned long)g.grid_segs * nplanes * nfields + 7) / 8 * 8 * C::SH;
+    } else {
+        g.grid_segs = (unsigned)((g.ncols + C::TC - 1) / C::TC);
+        ids = (unsigned long)g.grid_segs * nplanes * nfields;
+    }
+    g.grid_ids = (unsigned)ids;
+    return ids <= 0x7ffffffful;
+}
+
+#ifdef VFD_COLREC_TU
+// the launches of batches with records (FP32): col_rec_kernel
 template <typename T, int Q, int MODE, int RS, int V, int KS = KS_REAL, bool FOLD = false>
 static hipError_t col_go(const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
                          const void* tw, hipStream_t st) {
     using C = ColCfg<T, Q, V, RS>;
-    if constexpr (C::SH > 1) {
-        // grouped 1-D launch (col_kernel): 8 segment groups per 8 * SH ids
-        ColDesc g = cd;
-        g.grid_segs = (unsigned)((cd.ncols + C::TC_LINE - 1) / C::TC_LINE);
-        g.grid_planes = (unsigned)nplanes;
-        g.grid_fields = (unsigned)nfields;
-        const unsigned long groups = (unsigned long)g.grid_segs * nplanes * nfields;
-        const unsigned long ids = (groups + 7) / 8 * 8 * C::SH;
-        if (ids > 0x7fffffffu) return hipErrorInvalidConfiguration;
-        hipLaunchKernelGGL((col_kernel<T, Q, MODE, RS, V, KS, FOLD>), dim3((unsigned)ids), dim3(C::NT), 0, st, fields,
-                           g, (const cx<T>*)tw);
-    } else {
-        dim3 grid((unsigned)((cd.ncols + C::TC - 1) / C::TC), (unsigned)nplanes, (unsigned)nfields);
-        hipLaunchKernelGGL((col_kernel<T, Q, MODE, RS, V, KS, FOLD>), grid, dim3(C::NT), 0, st, fields, cd,
-                           (const cx<T>*)tw);
-    }
+    ColDesc g = cd;
+    if (!col_ids<C>(g, nfields, nplanes)) return hipErrorInvalidConfiguration;
+    // as many work-groups as the card holds, at most one per tile
+    static const int per_cu = blocks_per_cu(col_rec_kernel<Q, MODE, RS, V, KS, FOLD>, C::NT);
+    const unsigned cap = (unsigned)(num_cus() * per_cu);
+    hipLaunchKernelGGL((col_rec_kernel<Q, MODE, RS, V, KS, FOLD>), dim3(g.grid_ids < cap ? g.grid_ids : cap), dim3(C::NT), 0,
+                       st, fields, g, (const cx<T>*)tw);
     return hipGetLastError();
 }
+#else
+template <typename T, int Q, int MODE, int RS, int V, int KS = KS_REAL, bool FOLD = false>
+static hipError_t col_go(const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
+                         const void* tw, hipStream_t st) {
+    using C = ColCfg<T, Q, V, RS>;
+    ColDesc g = cd;
+    if (!col_ids<C>(g, nfields, nplanes)) return hipErrorInvalidConfiguration;
+    const dim3 grid = C::SH > 1 ? dim3(g.grid_ids) : dim3(g.grid_segs, (unsigned)nplanes, (unsigned)nfields);
+    hipLaunchKernelGGL((col_kernel<T, Q, MODE, RS, V, KS, FOLD>), grid, dim3(C::NT), 0, st, fields, g, (const cx<T>*)tw);
+    return hipGetLastError();
+}
+#endif
 
 // fused pass: the spectrum format picks the instantiation
 template <typename T, int Q, int RS, int V>
 static hipError_t col_fused(const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
                             const void* tw, hipStream_t st) {
     if (cd.kspec_sep) return col_go<T, Q, COL_FUSED, RS, V, KS_SEP>(fields, nfields, cd, nplanes, tw, st);
+#ifdef VFD_COLREC_TU
+    return hipErrorInvalidValue;  // records belong to separable tables
+#else
     if (cd.kspec_complex) return col_go<T, Q, COL_FUSED, RS, V, KS_COMPLEX>(fields, nfields, cd, nplanes, tw, st);
     return col_go<T, Q, COL_FUSED, RS, V, KS_REAL>(fields, nfields, cd, nplanes, tw, st);
+#endif
 }
 
 template <typename T, int Q, int V>
@@ -209,9 +235,17 @@ static hipError_t col_var(int variant, const FieldBatch& fields, int nfields, co
     }
 }
 
+#ifdef VFD_COLREC_TU
+hipError_t launch_col_rec(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes, const void* tw,
+                          hipStream_t st, int variant) {
+#else
 template <>
 hipError_t launch_col<VFD_REAL>(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd,
                                 long nplanes, const void* tw, hipStream_t st, int variant) {
+    if constexpr (sizeof(VFD_REAL) == 4) {
+        if (cd.records == RECORDS_FEW) return launch_col_rec(Q, fields, nfields, cd, nplanes, tw, st, variant);
+    }
+#endif
     constexpr bool kVariants = sizeof(VFD_REAL) == 4;  // FP64 has one schedule
     switch (Q) {
 #define VFD_HOT(QQ)                                                                     \

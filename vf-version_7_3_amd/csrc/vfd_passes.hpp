@@ -90,19 +90,23 @@ template <typename T> struct RowLds {
     __device__ __forceinline__ cx<T>& at(int n) { return base[n + (n >> 5)]; }
 };
 
-// Whether a field's tick goes through the direct convolution (vfd_direct.hpp):
-// the launches of the FFT passes then leave it alone.
-__device__ __forceinline__ bool dir_skip(const FieldDesc& fd) {
-    if (!fd.dir) return false;
-    const DirRecord* r = (const DirRecord*)fd.dir;
+// Whether a field's tick goes through the direct convolution (vfd_direct.hpp).
+__device__ __forceinline__ bool dir_form(const void* rec) {
+    const DirRecord* r = (const DirRecord*)rec;
     return r->ax[0].radius >= 0 && r->ax[1].radius >= 0 && r->ax[2].radius >= 0;
 }
 
-// The last item of `item`'s field in a work-group's sequence item, item + step,
-// ... (ngroups items per field): where its loop continues after a skipped field.
-__device__ __forceinline__ long field_end(long item, long ngroups, long step) {
-    const long left = (item / ngroups + 1) * ngroups - 1 - item;
-    return item + left / step * step;
+// The fields of a launch that the FFT passes do, as a bit mask: those whose
+// record does not have the direct form.  A lane reads a record.
+__device__ __forceinline__ unsigned fft_fields(const FieldBatch& fb, int nfields) {
+    const int l = (int)(threadIdx.x % 64u);
+    const bool fft = l < nfields && !dir_form(fb.f[l].dir);
+    return (unsigned)__ballot(fft);
+}
+// the n-th set bit of the mask (n < popcount)
+__device__ __forceinline__ unsigned nth_field(unsigned mask, unsigned n) {
+    for (; n; --n) mask &= mask - 1u;
+    return (unsigned)__builtin_ctz(mask);
 }
 
 // ------------------------------------------------------------- x forward
@@ -119,6 +123,14 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
     using O = typename B::O;
     __shared__ cx<T> smem[C::G * C::PITCH];
     __shared__ cx<T> twl[C::TW_N];
+    [[maybe_unused]] unsigned todo = ~0u;  // the launch's fields, where it has records
+    if constexpr (sizeof(T) == 4) {
+        if (g.records) {
+            todo = fft_fields(fb, nfields);
+            if (todo == 0) return;
+            nfields = __builtin_popcount(todo);
+        }
+    }
     const cx<T>* tw = twg;
     if constexpr (C::TW_LDS) {
         stage_table(twl, twg, 2 * L);
@@ -133,15 +145,12 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
     const bool cvf = g.pad_mode == PAD_CONSTANT_VF;
     constexpr unsigned RB = sizeof(T), CB = sizeof(cx<T>);
     for (long item = blockIdx.x; item < ngroups * nfields; item += gridDim.x) {
-        const int f = (int)(item / ngroups);
+        int f = (int)(item / ngroups);
+        if constexpr (sizeof(T) == 4) {
+            if (g.records) f = (int)nth_field(todo, (unsigned)f);
+        }
         const long row = (item % ngroups) * C::G + gr;
         const FieldDesc& fd = fb.f[f];
-        if constexpr (sizeof(T) == 4) {
-            if (dir_skip(fd)) {  // work-group uniform: on to the next field's groups
-                item = field_end(item, ngroups, gridDim.x);
-                continue;
-            }
-        }
         const auto rin = B::make(fd.in, g.in_bytes);
         const auto rwork = B::make(fd.work, g.work_bytes);
         const bool live = row < nrows;
@@ -227,6 +236,14 @@ xinv_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
     using O = typename B::O;
     __shared__ cx<T> smem[C::G * C::PITCH];
     __shared__ cx<T> twl[C::TW_N];
+    [[maybe_unused]] unsigned todo = ~0u;  // the launch's fields, where it has records
+    if constexpr (sizeof(T) == 4) {
+        if (g.records) {
+            todo = fft_fields(fb, nfields);
+            if (todo == 0) return;
+            nfields = __builtin_popcount(todo);
+        }
+    }
     const cx<T>* tw = twg;
     if constexpr (C::TW_LDS) {
         stage_table(twl, twg, 2 * L);
@@ -240,15 +257,12 @@ xinv_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
     RowLds<T> lds{smem + gr * C::PITCH};
     constexpr unsigned RB = sizeof(T), CB = sizeof(cx<T>);
     for (long item = blockIdx.x; item < ngroups * nfields; item += gridDim.x) {
-        const int f = (int)(item / ngroups);
+        int f = (int)(item / ngroups);
+        if constexpr (sizeof(T) == 4) {
+            if (g.records) f = (int)nth_field(todo, (unsigned)f);
+        }
         const long row = (item % ngroups) * C::G + gr;
         const FieldDesc& fd = fb.f[f];
-        if constexpr (sizeof(T) == 4) {
-            if (dir_skip(fd)) {
-                item = field_end(item, ngroups, gridDim.x);
-                continue;
-            }
-        }
         const auto rwork = B::make(fd.work, g.work_bytes);
         const auto rout = B::make(fd.out, g.out_bytes);
         const bool live = row < nrows;
@@ -434,9 +448,8 @@ template <typename T, int MODE, int NT> constexpr int col_waves_per_eu() {
 // Y_0[n] - W_P^-n Y_1[n].  Half the LDS per column of the unsplit transform:
 // twice the columns per tile.
 template <typename T, int Q, int MODE, int RS, int V, int KS = KS_REAL, bool FOLD = false>
-__global__ void __launch_bounds__((ColCfg<T, Q, V, RS>::NT))
-__attribute__((amdgpu_waves_per_eu((col_waves_per_eu<T, MODE, ColCfg<T, Q, V, RS>::NT>()))))
-col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
+__device__ __forceinline__ void col_tile(const FieldDesc& fd, const ColDesc& cd, const cx<T>* __restrict__ twg, unsigned bx,
+                                         unsigned by, unsigned tid) {
     static_assert(!FOLD || (RS == 2 && MODE == COL_INV), "folded split: RS = 2, inverse-only mode");
     using C = ColCfg<T, Q, V, RS>;
     using ShF = FftShape<T, Q, C::TPF, false, C::MAXR>;                // forward / inverse-only plan
@@ -449,40 +462,18 @@ col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
     __shared__ cx<T> tw[C::TW_N];
     constexpr bool SEP = MODE == COL_FUSED && KS == KS_SEP;
     __shared__ double gzs[SEP ? P : 1];  // separable: the gz table of the z frequencies
-    // Block coordinates.  Narrow tiles (SH of them share each 128-byte row
-    // segment) launch as a 1-D grid in which the SH tiles of one segment get
-    // work-group ids 8 apart.  Ids are dealt round-robin to the 8 XCDs, so the
-    // tiles sharing a line run side by side on one XCD and its L2 fetches the
-    // line once.
-    unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
-    if constexpr (C::SH > 1) {
-        const unsigned lin = blockIdx.x;
-        const unsigned grp = (lin / (8u * C::SH)) * 8u + lin % 8u;
-        const unsigned seg = grp % cd.grid_segs, rest = grp / cd.grid_segs;
-        bx = seg * C::SH + (lin / 8u) % C::SH;
-        by = rest % cd.grid_planes;
-        bz = rest / cd.grid_planes;
-        // whole-block exits, before any barrier: padding ids and tiles past the row end
-        if (bz >= cd.grid_fields || (long)bx * C::TC >= cd.ncols) return;
-    }
-    const FieldDesc& fd = fb.f[bz];
     if constexpr (SEP && sizeof(T) == 4) {
         // FP32 separable tables of radius <= kZDirectMaxR take the direct z pass
         // (zdirect_kernel, launched over the same fields); whole-block exit
         if (zform_of_table(fd.kspec, cd.kspec_bytes, cd.sep_g) != 0) return;
     }
     const auto rwork = B::make(fd.work, cd.work_bytes);
-    const int c = threadIdx.x % C::TC;
-    const int t = threadIdx.x / C::TC;
+    const int c = tid % C::TC;
+    const int t = tid / C::TC;
     const long col = (long)bx * C::TC + c;
     const bool live = col < cd.ncols;
     const O base = (O)((long)by * cd.pstride + col) * CB;
     const O rstep = (O)cd.rstride * CB;
-    if constexpr (sizeof(T) == 4) {
-        // whole-block exit; here, so that the other arguments are in flight
-        // with the record pointer
-        if (dir_skip(fd)) return;
-    }
     ColLds<T, C::TC> lds{smem + c};
     // non-temporal loads only when a tile row spans whole 128-byte lines: a
     // narrower tile (long columns) shares each line with its neighbours, which
@@ -681,6 +672,66 @@ col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
     }
 }
 
+// Block coordinates of id in a 1-D launch.  Narrow tiles (SH of them share each
+// 128-byte row segment) are always launched so, the SH tiles of one segment 8
+// ids apart: ids are dealt round-robin to the 8 XCDs, so the tiles sharing a
+// line run side by side on one XCD and its L2 fetches the line once.  False for
+// padding ids and tiles past the row end.
+template <typename C> __device__ __forceinline__ bool col_coords(const ColDesc& cd, unsigned id, unsigned nf, unsigned& bx, unsigned& by,
+                                            unsigned& bz) {
+    unsigned seg, rest;
+    if constexpr (C::SH > 1) {
+        const unsigned grp = (id / (8u * C::SH)) * 8u + id % 8u;
+        seg = grp % cd.grid_segs;
+        rest = grp / cd.grid_segs;
+        bx = seg * C::SH + (id / 8u) % C::SH;
+    } else {
+        bx = id % cd.grid_segs;
+        rest = id / cd.grid_segs;
+    }
+    by = rest % cd.grid_planes;
+    bz = rest / cd.grid_planes;
+    return bz < nf && (long)bx * C::TC < cd.ncols;
+}
+
+template <typename T, int Q, int MODE, int RS, int V, int KS = KS_REAL, bool FOLD = false>
+__global__ void __launch_bounds__((ColCfg<T, Q, V, RS>::NT))
+__attribute__((amdgpu_waves_per_eu((col_waves_per_eu<T, MODE, ColCfg<T, Q, V, RS>::NT>()))))
+col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
+    using C = ColCfg<T, Q, V, RS>;
+    unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+    if constexpr (C::SH > 1)
+        if (!col_coords<C>(cd, blockIdx.x, cd.grid_fields, bx, by, bz)) return;
+    if constexpr (sizeof(T) == 4) {
+        if (cd.records && dir_form(fb.f[bz].dir)) return;  // not the FFT passes' field
+    }
+    col_tile<T, Q, MODE, RS, V, KS, FOLD>(fb.f[bz], cd, twg, bx, by, threadIdx.x);
+}
+
+// The same pass for batches that are expected to have few or no fields of the
+// FFT form (RECORDS_FEW): a persistent 1-D launch walking the tiles of those
+// fields, so that a batch without any costs the launch and nothing per tile
+// (col_kernel's one work-group per tile: 0.29 ms of passes in a 2.1 ms tick of 8
+// fields 1024x512x128, 40 of 242 us at 301x187x75).  It runs tiles slower than
+// col_kernel (loop-carried registers, one tile's stores before the next one's
+// loads: 13.6 against 11.7 ms for a tick of 8 FFT-form fields 1024x512x128).
+template <int Q, int MODE, int RS, int V, int KS, bool FOLD>
+__global__ void __launch_bounds__((ColCfg<float, Q, V, RS>::NT))
+__attribute__((amdgpu_waves_per_eu((col_waves_per_eu<float, MODE, ColCfg<float, Q, V, RS>::NT>()))))
+col_rec_kernel(const FieldBatch fb, ColDesc cd, const float2* __restrict__ twg) {
+    using C = ColCfg<float, Q, V, RS>;
+    const unsigned todo = fft_fields(fb, (int)cd.grid_fields);
+    const unsigned nf = (unsigned)__builtin_popcount(todo);
+    if (nf == 0) return;
+    for (unsigned id = blockIdx.x; id < cd.grid_ids; id += gridDim.x) {
+        unsigned bx, by, bz, tid = threadIdx.x;
+        if (!col_coords<C>(cd, id, nf, bx, by, bz)) continue;
+        asm volatile("" : "+v"(tid));  // nothing of one tile is kept in registers for the next
+        col_tile<float, Q, MODE, RS, V, KS, FOLD>(fb.f[nth_field(todo, bz)], cd, twg, bx, by, tid);
+        __syncthreads();  // the tile's LDS is read
+    }
+}
+
 // ------------------------------------------------ z pass, direct form (FP32)
 // With the separable spectrum the z factor gz is the DFT, on the Pz box, of
 // the normalized window g_j (|j| <= R).  Multiplying by gz between the forward
@@ -700,7 +751,7 @@ col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
 // in no class of the launch (zform_of) exits at once.
 
 template <int RM>
-__device__ __forceinline__ void zdirect_column(const FieldDesc& fd, const ColDesc& cd) {
+__device__ __forceinline__ void zdirect_column(const FieldDesc& fd, const ColDesc& cd, unsigned bx, unsigned by) {
     using B = BufOps<float>;
     using O = typename B::O;
     using BD = BufOps<double>;
@@ -708,8 +759,8 @@ __device__ __forceinline__ void zdirect_column(const FieldDesc& fd, const ColDes
     constexpr int U = 2 * RM + 1;
     constexpr unsigned CB = sizeof(cx<float>);
     const auto rwork = B::make(fd.work, cd.work_bytes);
-    const long col = (long)blockIdx.x * 64 + threadIdx.x;
-    const long ky = blockIdx.y;
+    const long col = (long)bx * 64 + threadIdx.x;
+    const long ky = by;
     const bool live = col < cd.ncols;
     const O base = (O)((live ? ky * cd.pstride + col : 0) * CB);
     const O rstep = (O)cd.rstride * CB;
@@ -760,7 +811,7 @@ __device__ __forceinline__ void zdirect_column(const FieldDesc& fd, const ColDes
     // columns past the row's end (the last one, 1025 = 16 * 64 + 1 columns on
     // a 2048 box) goes through the L2: a narrow non-temporal store costs a
     // partial-line write to HBM (this form is 8 % faster at radius 16).
-    if ((long)(blockIdx.x + 1) * 64 <= cd.ncols) body(std::integral_constant<int, kStream>{});
+    if ((long)(bx + 1) * 64 <= cd.ncols) body(std::integral_constant<int, kStream>{});
     else body(std::integral_constant<int, kCacheDefault>{});
 }
 

@@ -233,7 +233,8 @@ int plan_init(const vfd_plan_desc* d, Plan* p) {
                          q.work_bytes, q.kspec_bytes, q.field_bytes);
     // the direct-convolution form (vfd_direct.hpp): its record follows the FFT
     // passes' work array, whose front holds the pass between x-y and z
-    q.direct = q.prec == VFD_F32 && q.kspec_format == VFD_KSPEC_SEPARABLE;
+    q.direct = q.prec == VFD_F32 && q.kspec_format == VFD_KSPEC_SEPARABLE &&
+               std::max({q.px, q.py, q.pz}) / 2 <= kDirHalfMax;
     if (q.direct) {
         q.rec_off = round_up((long)std::max(q.work_bytes, q.field_bytes), 256);
         q.work_bytes = q.rec_off + kDirRecordBytes;
@@ -363,7 +364,11 @@ template <typename T>
 static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pass_lo, int pass_hi,
                     hipStream_t st, const Epilogue* epi, int zpart = -1, Form form = Form::by_table,
                     int max_radius = kDirMaxR) {
-    const bool records = p.direct && form != Form::fft;
+    // only tables of the direct form's radius so far: the FFT passes are
+    // expected to have nothing to do (tables can come from elsewhere)
+    const int records = !p.direct || form == Form::fft                          ? RECORDS_NONE
+                        : __atomic_load_n(&p.tables, __ATOMIC_RELAXED) == 1 ? RECORDS_FEW
+                                                                             : RECORDS_MANY;
     for (int f0 = 0; f0 < nfields; f0 += kMaxFieldsPerLaunch) {
         const int nf = std::min(kMaxFieldsPerLaunch, nfields - f0);
         FieldBatch fb;
@@ -390,11 +395,12 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
         const size_t work_bytes = p.direct ? p.rec_off : p.work_bytes;  // without the record
         GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, p.pad_mode, p.kspec_format == VFD_KSPEC_COMPLEX_STD,
                    p.field_bytes, work_bytes, p.kspec_bytes, p.field_bytes,
-                   p.kspec_format == VFD_KSPEC_COMPLEX_STD ? 1.0 : (double)p.px * p.py * p.pz};
+                   p.kspec_format == VFD_KSPEC_COMPLEX_STD ? 1.0 : (double)p.px * p.py * p.pz, records};
         ColDesc y{};
         y.mode = COL_FWD; y.rs = p.rs_y; y.nin = p.ny; y.nout = p.py; y.ncols = p.hx;
         y.rstride = p.ld; y.pstride = p.plane; y.scale = 1.0;
         y.work_bytes = work_bytes; y.kspec_bytes = p.kspec_bytes;
+        y.records = records;
         ColDesc z{};
         z.mode = COL_FUSED; z.rs = p.rs_z; z.nin = p.nz; z.nout = p.nz; z.ncols = p.hx;
         z.rstride = p.plane; z.pstride = p.ld; z.ks_row = p.ks_row; z.ks_plane = p.ks_plane;
@@ -406,6 +412,7 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
         // the real native spectrum carries the 1/(px py pz) normalization
         z.scale = z.kspec_complex ? 1.0 / ((double)p.px * p.py * p.pz) : 1.0;
         z.work_bytes = work_bytes; z.kspec_bytes = p.kspec_bytes;
+        z.records = records;
         ColDesc yi = y;
         yi.mode = COL_INV; yi.nin = p.py; yi.nout = p.ny;
         if (p.fold_y) { yi.rs = 2; yi.fold = 1; }
@@ -563,6 +570,7 @@ int plan_autotune(Plan& p, int nfields, hipStream_t st, float* best_ms) {
     if (int rc = hip_check(hipMalloc((void**)&buf, total), "autotune scratch")) return rc;
     hipLaunchKernelGGL(scratch_fill_kernel, dim3(2048), dim3(256), 0, st, (unsigned*)buf, total / 4, 0x5EEDu);
     int rc = hip_check(hipGetLastError(), "autotune fill");
+    const int tables = p.tables;
     std::vector<vfd_field> fl(nfields);
     for (int i = 0; i < nfields; ++i) {
         char* f = buf + (size_t)i * per_field;
@@ -582,6 +590,7 @@ int plan_autotune(Plan& p, int nfields, hipStream_t st, float* best_ms) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (!rc) rc = hip_check(hipEventCreate(&e0), "event");
     if (!rc) rc = hip_check(hipEventCreate(&e1), "event");
+    p.tables = tables;  // the scratch tables say nothing about the plan's use
     const int saved[5] = {p.var[0], p.var[1], p.var[2], p.var[3], p.var[4]};
     // a variant is timed inside whole steps (the pass between events, the
     // other passes around it): a pass repeated on its own meets the caches in
@@ -638,7 +647,7 @@ static int run_r2c(const Plan& p, const void* in, void* out, hipStream_t st) {
     fb.f[0].in = in;
     fb.f[0].work = out;
     const size_t cbytes = (size_t)p.pz * p.py * p.hx * 2 * p.prec;
-    GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, VFD_PAD_ZERO, 0, p.field_bytes, cbytes, 0, 0, 1.0};
+    GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, VFD_PAD_ZERO, 0, p.field_bytes, cbytes, 0, 0, 1.0, 0};
     hipError_t e = launch_xfwd<T>(p.L, fb, 1, g, p.tw_x, st);
     if (e != hipSuccess) return hip_check(e, "r2c x launch");
     ColDesc y{};
@@ -670,7 +679,7 @@ static int run_c2r(const Plan& p, void* in, void* out, hipStream_t st) {
     y.nin = p.py; y.nout = p.py; y.rstride = p.ld; y.pstride = p.plane;
     e = launch_col<T>(p.py, fb, 1, y, p.nz, p.tw_y, st);
     if (e != hipSuccess) return hip_check(e, "c2r y launch");
-    GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, VFD_PAD_ZERO, 0, 0, cbytes, 0, p.field_bytes, 1.0};
+    GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, VFD_PAD_ZERO, 0, 0, cbytes, 0, p.field_bytes, 1.0, 0};
     e = launch_xinv<T>(p.L, fb, 1, g, p.tw_x, st);
     return e == hipSuccess ? VFD_OK : hip_check(e, "c2r x launch");
 }
@@ -761,6 +770,7 @@ int plan_gauss_spectrum(const Plan& p, double sigma2, double decay, void* d_kspe
                            "gauss tables upload");
         // the host vector must outlive the async copy
         if (!rc) rc = hip_check(hipStreamSynchronize(st), "gauss tables sync");
+        if (!rc) __atomic_fetch_or(&p.tables, R <= kDirMaxR ? 1 : 2, __ATOMIC_RELAXED);
         return rc;
     }
     double* d = nullptr;

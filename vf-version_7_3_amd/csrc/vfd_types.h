@@ -9,6 +9,11 @@ enum PadMode { PAD_CONSTANT_VF = 3, PAD_ZERO = 100 };
 
 enum ColMode { COL_FWD = 0, COL_INV = 1, COL_FUSED = 2 };
 
+// Whether the fields of an FFT pass carry DirRecords (FieldDesc::dir), and how
+// many of them are expected to be of the FFT form: that picks between launches of
+// one work-group per tile and persistent ones that leave early, not the result.
+enum Records { RECORDS_NONE = 0, RECORDS_MANY = 1, RECORDS_FEW = 2 };
+
 // Per-field pointers of one launch.
 struct FieldDesc {
     const void* in;     // real field [Nz][Ny][Nx] (x-forward input)
@@ -24,8 +29,8 @@ struct FieldDesc {
     float* vis;         //   min(t * vis_scale, 1) into a dense [Nz/s][Ny/s][Nx/s] array
     float vis_scale;
     int pad2_;
-    // FP32 separable fields: the field's DirRecord; a launch of the FFT passes
-    // skips a field whose record has the direct form (null: no record, FFT form)
+    // FP32 separable fields: the field's DirRecord (read by the direct form's
+    // launches and, where GridDesc / ColDesc::records is set, by the FFT passes')
     const void* dir;
 };
 
@@ -49,6 +54,7 @@ struct GridDesc {
     // is stored unnormalized (1), the real one with 1/(Px Py Pz) folded in
     // (Px Py Pz)
     double kdc_scale;
+    int records;        // Records: fields of the direct form are left out
 };
 
 // One column pass (y or z).
@@ -69,6 +75,8 @@ struct ColDesc {
     // grouped 1-D launch of narrow tiles (set by the launcher): planes and
     // fields of the launch, 128-byte row segments per plane row
     unsigned grid_planes, grid_fields, grid_segs;
+    unsigned grid_ids;  // ids of a 1-D launch (grid_segs = tiles per row where tiles are not narrow)
+    int records;        // Records: fields of the direct form are left out
     int sep_g;          // separable: table offset (elements) of [R | g_0 .. g_kZDirectMaxR]
     int fold;           // rs = 2 with output rows past P/2 (FP32 inverse-only, fold_supported)
 };
@@ -96,6 +104,7 @@ struct XlDesc {
 // Windows up to kDirMaxR take it; its cost grows with 2 R + 1 per axis, and at
 // R = 31 it is still a fraction of the FFT passes' time.
 constexpr int kDirMaxR = 31;
+constexpr int kDirHalfMax = 2304;  // half the longest box axis (dir_classify's LDS): the longest compiled length
 struct DirAxis {
     double gain;               // exact window sum / sum of the FP32 taps (1 where not all taps are >= 0)
     int radius;                // -1: the axis' table is not a short window
