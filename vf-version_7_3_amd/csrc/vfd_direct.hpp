@@ -22,6 +22,10 @@
 
 namespace vfd {
 
+__device__ __forceinline__ DirRecord* dir_record(const FieldDesc& fd, const DirDims& d) {
+    return d.rec_off < 0 ? (DirRecord*)const_cast<void*>(fd.kspec) : (DirRecord*)((char*)fd.work + d.rec_off);
+}
+
 // --------------------------------------------------------------- classify
 // One work-group per (axis, field): the axis' table t[k] (x: the half k <= P/2;
 // y, z: all P entries) back to its window,
@@ -48,7 +52,7 @@ dir_classify_kernel(const FieldBatch fb, DirDims d) {
     const int ax = blockIdx.x;
     const FieldDesc& fd = fb.f[blockIdx.y];
     const double* tab = (const double*)fd.kspec;
-    DirRecord* rec = (DirRecord*)fd.dir;
+    DirRecord* rec = dir_record(fd, d);
     const int P = ax == 0 ? d.px : ax == 1 ? d.py : d.pz;
     const int n = ax == 0 ? d.nx : ax == 1 ? d.ny : d.nz;
     const double* t = tab + 1 + (ax == 0 ? 0 : ax == 1 ? d.px / 2 + 1 : d.px / 2 + 1 + d.py);
@@ -254,7 +258,25 @@ __device__ __forceinline__ void dir_xy_strip(float* lds, const DirRecord* rec, r
     const int nb = M0 + (y1 - y0 + B - 1) / B;
     const unsigned plane = (unsigned)z * (unsigned)d.ny * (unsigned)d.nx;
     float4 q[NLD];
+    // element offset of each chunk from the batch's first row, columns outside
+    // the data (whole 16-byte chunks on the left, the row's end on the right)
+    // masked once; where the whole batch is inside the chunk of rows a load is
+    // this offset and the wave's scalar base
+    unsigned voff[NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+        const int idx = tid + i * kDirThreads, r = idx / W4, x = x0 - RB4 + 4 * (idx % W4);
+        voff[i] = (NLD * kDirThreads == B * W4 || r < B) && x >= 0 && x + 4 <= d.nx ? ((unsigned)(r * d.nx + x)) * 4u : kBufOOB;
+    }
+    const bool cut = x0 + TX + RB4 > d.nx && d.nx % 4 != 0;  // a chunk of the strip crosses the row's end
     auto fetch = [&](int yb) {
+        if (yb >= ylo && yb + B <= yhi && !cut) {
+            const int base = __builtin_amdgcn_readfirstlane((int)((plane + (unsigned)yb * (unsigned)d.nx) * 4u));
+#pragma unroll
+            for (int i = 0; i < NLD; ++i)
+                q[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rin, voff[i], base, kCacheDefault));
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int idx = tid + i * kDirThreads, r = idx / W4, c = idx % W4;
@@ -266,6 +288,7 @@ __device__ __forceinline__ void dir_xy_strip(float* lds, const DirRecord* rec, r
     };
     const int xr = tid / (TX / 8), xt = tid % (TX / 8);          // x phase: row of the batch, 8 columns
     const int col = tid % TX, rg = __builtin_amdgcn_readfirstlane(tid / TX);  // y phase: column, 8 rows
+    const unsigned xoff = x0 + col < d.nx ? (unsigned)(x0 + col) * 4u : kBufOOB;
     int pos = 0;  // ring row of the batch's first row
     fetch(yb);
     for (int b = 0; b < nb; ++b) {
@@ -298,12 +321,14 @@ __device__ __forceinline__ void dir_xy_strip(float* lds, const DirRecord* rec, r
             start = start < 0 ? start + RS : start >= RS ? start - RS : start;
             DirSums acc;
             dir_ring_conv<TX, RB>(acc, ty, ring, start, col);
-            const int yo = yb - RB4 + 8 * rg, x = x0 + col;
-            unsigned off = (plane + (unsigned)yo * (unsigned)d.nx + (unsigned)x) * 4u;
+            const int yo = yb - RB4 + 8 * rg;  // wave-uniform, as the rows' bases
+            unsigned base = (plane + (unsigned)yo * (unsigned)d.nx) * 4u;
 #pragma unroll
             for (int v = 0; v < kDirOut; ++v) {
-                BufOps<float>::st_r(acc[v], rw, x < d.nx && yo + v < y1 ? off : kBufOOB);
-                off += (unsigned)d.nx * 4u;
+                if (yo + v < y1)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[v]), rw, xoff, (int)base,
+                                                          kCacheDefault);
+                base += (unsigned)d.nx * 4u;
             }
         }
         yb += B;
@@ -334,8 +359,8 @@ __global__ void __launch_bounds__(kDirThreads) dir_xy_kernel(const FieldBatch fb
     const unsigned ch = rest % d.ychunks, f = rest / d.ychunks;
     if (f >= d.nfields) return;  // padding ids
     const FieldDesc& fd = fb.f[f];
-    const DirRecord* rec = (const DirRecord*)fd.dir;
-    if (!dir_form(fd.dir)) return;  // the FFT passes do it
+    const DirRecord* rec = dir_record(fd, d);
+    if (!dir_form(rec)) return;  // the FFT passes do it
     const int R = __builtin_amdgcn_readfirstlane(max(rec->ax[0].radius, rec->ax[1].radius));
     const rsrc_t rin = make_rsrc(fd.in, d.bytes), rw = make_rsrc(fd.work, d.bytes);
     const int x0 = (int)tile * TX, y0 = (int)ch * d.yrows, y1 = min(d.ny, y0 + d.yrows);
@@ -449,8 +474,8 @@ template <int TX, bool VIS, int POL>
 __global__ void __launch_bounds__(kDirThreads) dir_z_kernel(const FieldBatch fb, DirDims d) {
     extern __shared__ __align__(16) float dir_lds[];
     const FieldDesc& fd = fb.f[blockIdx.y];
-    const DirRecord* rec = (const DirRecord*)fd.dir;
-    if (!dir_form(fd.dir)) return;  // the FFT passes do it
+    const DirRecord* rec = dir_record(fd, d);
+    if (!dir_form(rec)) return;  // the FFT passes do it
     const int R = __builtin_amdgcn_readfirstlane(rec->ax[2].radius);
     if (R > d.max_radius) return;
 #define VFD_GO(RB) \

@@ -10,7 +10,7 @@ namespace vfd {
 __global__ void __launch_bounds__(64) zdirect_kernel(const FieldBatch fb, ColDesc cd, unsigned classes) {
     unsigned id = blockIdx.x, nf = cd.grid_fields, todo = ~0u;
     if (cd.records) {
-        todo = fft_fields(fb, (int)nf);
+        todo = fft_fields(fb, (int)nf, cd.rec_off);
         nf = (unsigned)__builtin_popcount(todo);
         if (nf == 0) return;
     }

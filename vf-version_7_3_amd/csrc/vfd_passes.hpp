@@ -98,9 +98,9 @@ __device__ __forceinline__ bool dir_form(const void* rec) {
 
 // The fields of a launch that the FFT passes do, as a bit mask: those whose
 // record does not have the direct form.  A lane reads a record.
-__device__ __forceinline__ unsigned fft_fields(const FieldBatch& fb, int nfields) {
+__device__ __forceinline__ unsigned fft_fields(const FieldBatch& fb, int nfields, unsigned long rec_off) {
     const int l = (int)(threadIdx.x % 64u);
-    const bool fft = l < nfields && !dir_form(fb.f[l].dir);
+    const bool fft = l < nfields && !dir_form((const char*)fb.f[l].work + rec_off);
     return (unsigned)__ballot(fft);
 }
 // the n-th set bit of the mask (n < popcount)
@@ -126,7 +126,7 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
     [[maybe_unused]] unsigned todo = ~0u;  // the launch's fields, where it has records
     if constexpr (sizeof(T) == 4) {
         if (g.records) {
-            todo = fft_fields(fb, nfields);
+            todo = fft_fields(fb, nfields, g.rec_off);
             if (todo == 0) return;
             nfields = __builtin_popcount(todo);
         }
@@ -239,7 +239,7 @@ xinv_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
     [[maybe_unused]] unsigned todo = ~0u;  // the launch's fields, where it has records
     if constexpr (sizeof(T) == 4) {
         if (g.records) {
-            todo = fft_fields(fb, nfields);
+            todo = fft_fields(fb, nfields, g.rec_off);
             if (todo == 0) return;
             nfields = __builtin_popcount(todo);
         }
@@ -703,7 +703,7 @@ col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
     if constexpr (C::SH > 1)
         if (!col_coords<C>(cd, blockIdx.x, cd.grid_fields, bx, by, bz)) return;
     if constexpr (sizeof(T) == 4) {
-        if (cd.records && dir_form(fb.f[bz].dir)) return;  // not the FFT passes' field
+        if (cd.records && dir_form((const char*)fb.f[bz].work + cd.rec_off)) return;  // not the FFT passes' field
     }
     col_tile<T, Q, MODE, RS, V, KS, FOLD>(fb.f[bz], cd, twg, bx, by, threadIdx.x);
 }
@@ -720,7 +720,7 @@ __global__ void __launch_bounds__((ColCfg<float, Q, V, RS>::NT))
 __attribute__((amdgpu_waves_per_eu((col_waves_per_eu<float, MODE, ColCfg<float, Q, V, RS>::NT>()))))
 col_rec_kernel(const FieldBatch fb, ColDesc cd, const float2* __restrict__ twg) {
     using C = ColCfg<float, Q, V, RS>;
-    const unsigned todo = fft_fields(fb, (int)cd.grid_fields);
+    const unsigned todo = fft_fields(fb, (int)cd.grid_fields, cd.rec_off);
     const unsigned nf = (unsigned)__builtin_popcount(todo);
     if (nf == 0) return;
     for (unsigned id = blockIdx.x; id < cd.grid_ids; id += gridDim.x) {

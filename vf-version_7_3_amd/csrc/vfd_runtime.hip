@@ -351,12 +351,13 @@ static int run_xlast(const Plan& p, const FieldBatch& fb, int nf, int pass_lo, i
     return VFD_OK;
 }
 
-static DirDims dir_dims(const Plan& p, int max_radius) {
+static DirDims dir_dims(const Plan& p, int max_radius, long rec_off) {
     DirDims d{};
     d.nx = p.nx; d.ny = p.ny; d.nz = p.nz;
     d.px = p.px; d.py = p.py; d.pz = p.pz;
     d.max_radius = max_radius;
     d.bytes = p.field_bytes;
+    d.rec_off = rec_off;
     return d;
 }
 
@@ -381,7 +382,6 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
             fb.f[i].kspec = f.kspec;
             fb.f[i].base = f.base;
             fb.f[i].epi = f.epi;
-            if (records) fb.f[i].dir = form == Form::direct ? f.kspec : (char*)f.work + p.rec_off;
             if (epi && epi->deltas) {
                 fb.f[i].delta = epi->deltas[f0 + i];
                 fb.f[i].decay = epi->decay[f0 + i];
@@ -395,12 +395,12 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
         const size_t work_bytes = p.direct ? p.rec_off : p.work_bytes;  // without the record
         GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, p.pad_mode, p.kspec_format == VFD_KSPEC_COMPLEX_STD,
                    p.field_bytes, work_bytes, p.kspec_bytes, p.field_bytes,
-                   p.kspec_format == VFD_KSPEC_COMPLEX_STD ? 1.0 : (double)p.px * p.py * p.pz, records};
+                   p.kspec_format == VFD_KSPEC_COMPLEX_STD ? 1.0 : (double)p.px * p.py * p.pz, records, p.rec_off};
         ColDesc y{};
         y.mode = COL_FWD; y.rs = p.rs_y; y.nin = p.ny; y.nout = p.py; y.ncols = p.hx;
         y.rstride = p.ld; y.pstride = p.plane; y.scale = 1.0;
         y.work_bytes = work_bytes; y.kspec_bytes = p.kspec_bytes;
-        y.records = records;
+        y.records = records; y.rec_off = p.rec_off;
         ColDesc z{};
         z.mode = COL_FUSED; z.rs = p.rs_z; z.nin = p.nz; z.nout = p.nz; z.ncols = p.hx;
         z.rstride = p.plane; z.pstride = p.ld; z.ks_row = p.ks_row; z.ks_plane = p.ks_plane;
@@ -412,7 +412,7 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
         // the real native spectrum carries the 1/(px py pz) normalization
         z.scale = z.kspec_complex ? 1.0 / ((double)p.px * p.py * p.pz) : 1.0;
         z.work_bytes = work_bytes; z.kspec_bytes = p.kspec_bytes;
-        z.records = records;
+        z.records = records; z.rec_off = p.rec_off;
         ColDesc yi = y;
         yi.mode = COL_INV; yi.nin = p.py; yi.nout = p.ny;
         if (p.fold_y) { yi.rs = 2; yi.fold = 1; }
@@ -425,7 +425,7 @@ static int run_tick(const Plan& p, const vfd_field* fields, int nfields, int pas
         }
         // The direct form's x-y pass goes with the first pass of the FFT form and
         // its z pass with the last: in between it is the FFT fields' work alone.
-        const DirDims dd = dir_dims(p, max_radius);
+        const DirDims dd = dir_dims(p, max_radius, form == Form::direct ? -1 : (long)p.rec_off);
         for (int pass = pass_lo; pass < pass_hi; ++pass) {
             hipError_t e = hipSuccess;
             if constexpr (sizeof(T) == 4) {
@@ -481,8 +481,8 @@ int plan_direct_record(const Plan& p, const void* d_kspec, void* rec, int* radiu
     FieldBatch fb;
     memset(&fb, 0, sizeof fb);
     fb.f[0].kspec = d_kspec;
-    fb.f[0].dir = rec;
-    if (int rc = hip_check(launch_dir_classify(fb, 1, dir_dims(p, kDirMaxR), st), "classify launch")) return rc;
+    fb.f[0].work = rec;
+    if (int rc = hip_check(launch_dir_classify(fb, 1, dir_dims(p, kDirMaxR, 0), st), "classify launch")) return rc;
     DirRecord h;
     if (int rc = hip_check(hipMemcpyAsync(&h, rec, sizeof h, hipMemcpyDeviceToHost, st), "record download")) return rc;
     if (int rc = hip_check(hipStreamSynchronize(st), "record sync")) return rc;
@@ -647,7 +647,7 @@ static int run_r2c(const Plan& p, const void* in, void* out, hipStream_t st) {
     fb.f[0].in = in;
     fb.f[0].work = out;
     const size_t cbytes = (size_t)p.pz * p.py * p.hx * 2 * p.prec;
-    GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, VFD_PAD_ZERO, 0, p.field_bytes, cbytes, 0, 0, 1.0, 0};
+    GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, VFD_PAD_ZERO, 0, p.field_bytes, cbytes, 0, 0, 1.0, 0, 0};
     hipError_t e = launch_xfwd<T>(p.L, fb, 1, g, p.tw_x, st);
     if (e != hipSuccess) return hip_check(e, "r2c x launch");
     ColDesc y{};
@@ -679,7 +679,7 @@ static int run_c2r(const Plan& p, void* in, void* out, hipStream_t st) {
     y.nin = p.py; y.nout = p.py; y.rstride = p.ld; y.pstride = p.plane;
     e = launch_col<T>(p.py, fb, 1, y, p.nz, p.tw_y, st);
     if (e != hipSuccess) return hip_check(e, "c2r y launch");
-    GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, VFD_PAD_ZERO, 0, 0, cbytes, 0, p.field_bytes, 1.0, 0};
+    GridDesc g{p.nx, p.ny, p.nz, p.L, p.ld, p.plane, VFD_PAD_ZERO, 0, 0, cbytes, 0, p.field_bytes, 1.0, 0, 0};
     e = launch_xinv<T>(p.L, fb, 1, g, p.tw_x, st);
     return e == hipSuccess ? VFD_OK : hip_check(e, "c2r x launch");
 }

@@ -9,7 +9,7 @@ enum PadMode { PAD_CONSTANT_VF = 3, PAD_ZERO = 100 };
 
 enum ColMode { COL_FWD = 0, COL_INV = 1, COL_FUSED = 2 };
 
-// Whether the fields of an FFT pass carry DirRecords (FieldDesc::dir), and how
+// Whether the fields of an FFT pass carry DirRecords (in work, at rec_off), and how
 // many of them are expected to be of the FFT form: that picks between launches of
 // one work-group per tile and persistent ones that leave early, not the result.
 enum Records { RECORDS_NONE = 0, RECORDS_MANY = 1, RECORDS_FEW = 2 };
@@ -29,9 +29,6 @@ struct FieldDesc {
     float* vis;         //   min(t * vis_scale, 1) into a dense [Nz/s][Ny/s][Nx/s] array
     float vis_scale;
     int pad2_;
-    // FP32 separable fields: the field's DirRecord (read by the direct form's
-    // launches and, where GridDesc / ColDesc::records is set, by the FFT passes')
-    const void* dir;
 };
 
 // Fields of one launch, passed by value as a kernel argument (graph-capture
@@ -55,6 +52,7 @@ struct GridDesc {
     // (Px Py Pz)
     double kdc_scale;
     int records;        // Records: fields of the direct form are left out
+    unsigned long rec_off;
 };
 
 // One column pass (y or z).
@@ -77,6 +75,7 @@ struct ColDesc {
     unsigned grid_planes, grid_fields, grid_segs;
     unsigned grid_ids;  // ids of a 1-D launch (grid_segs = tiles per row where tiles are not narrow)
     int records;        // Records: fields of the direct form are left out
+    unsigned long rec_off;
     int sep_g;          // separable: table offset (elements) of [R | g_0 .. g_kZDirectMaxR]
     int fold;           // rs = 2 with output rows past P/2 (FP32 inverse-only, fold_supported)
 };
@@ -124,6 +123,7 @@ struct DirDims {
     int yrows;                 // rows per chunk
     int max_radius;            // largest radius the launch's LDS holds
     unsigned long bytes;       // of one real field
+    long rec_off;              // the records: work + rec_off, or kspec itself where negative
 };
 
 // Largest window radius the direct z pass takes (separable spectrum, FP32);
