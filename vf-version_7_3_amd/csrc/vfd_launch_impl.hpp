@@ -182,7 +182,13 @@ static hipError_t col_go(const FieldBatch& fields, int nfields, const ColDesc& c
     using C = ColCfg<T, Q, V, RS>;
     ColDesc g = cd;
     if (!col_ids<C>(g, nfields, nplanes)) return hipErrorInvalidConfiguration;
-    const dim3 grid = C::SH > 1 ? dim3(g.grid_ids) : dim3(g.grid_segs, (unsigned)nplanes, (unsigned)nfields);
+    dim3 grid = C::SH > 1 ? dim3(g.grid_ids) : dim3(g.grid_segs, (unsigned)nplanes, (unsigned)nfields);
+    if constexpr (KS == KS_ROWS) {  // every tile by itself, whole rounds of XCDs
+        g.grid_segs = (unsigned)((cd.ncols + C::TC - 1) / C::TC);
+        const unsigned long ids = ((unsigned long)g.grid_segs * nplanes * nfields + 7) / 8 * 8;
+        if (ids > 0x7fffffffu) return hipErrorInvalidConfiguration;
+        grid = dim3((unsigned)ids);
+    }
     hipLaunchKernelGGL((col_kernel<T, Q, MODE, RS, V, KS, FOLD>), grid, dim3(C::NT), 0, st, fields, g, (const cx<T>*)tw);
     return hipGetLastError();
 }
@@ -212,6 +218,14 @@ static hipError_t col_mode(const FieldBatch& fields, int nfields, const ColDesc&
         return hipErrorInvalidValue;
     }
     const int key = cd.mode * 2 + (cd.rs - 1);
+#ifndef VFD_COLREC_TU
+    if (cd.off_lines && cd.rs == 1 && cd.mode != COL_FUSED) {
+        // one schedule, that of the lengths compiled in one
+        constexpr int VR = single_var<T, Q>();
+        if (cd.mode == COL_FWD) return col_go<T, Q, COL_FWD, 1, VR, KS_ROWS>(fields, nfields, cd, nplanes, tw, st);
+        return col_go<T, Q, COL_INV, 1, VR, KS_ROWS>(fields, nfields, cd, nplanes, tw, st);
+    }
+#endif
     switch (key) {
         case COL_FWD * 2 + 0: return col_go<T, Q, COL_FWD, 1, V>(fields, nfields, cd, nplanes, tw, st);
         case COL_FWD * 2 + 1: return col_go<T, Q, COL_FWD, 2, V>(fields, nfields, cd, nplanes, tw, st);

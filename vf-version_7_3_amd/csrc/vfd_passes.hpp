@@ -38,6 +38,9 @@ template <typename T, int Q, int V = 0> struct RowCfg {
     static constexpr int G = (NTT / TPF) > 0 ? (NTT / TPF) : 1;     // rows per group
     static constexpr int NT = TPF * G;
     static constexpr int PITCH = Q + Q / 32 + 1;                 // padded LDS row (RowLds)
+    // a row's lanes touch TPF adjacent elements at a time: non-temporal where that
+    // is a whole 128-byte line, through the L2 (which merges them) where it is not
+    static constexpr int POL = TPF * (int)sizeof(cx<T>) >= 128 ? kStream : kCacheDefault;
     // each row's transform and LDS row belong to one wavefront: its stages
     // synchronize that wave alone (stage_sync)
     static constexpr bool WS = wave_local<TPF>();
@@ -144,6 +147,7 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
     RowLds<T> lds{smem + gr * C::PITCH};
     const bool cvf = g.pad_mode == PAD_CONSTANT_VF;
     constexpr unsigned RB = sizeof(T), CB = sizeof(cx<T>);
+    constexpr int NTX = C::POL;
     for (long item = blockIdx.x; item < ngroups * nfields; item += gridDim.x) {
         int f = (int)(item / ngroups);
         if constexpr (sizeof(T) == 4) {
@@ -175,15 +179,15 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
                 if (vec) {
                     // the pair in one load; the constant pad's faces are cut afterwards
                     const bool ok = n >= 0 && row_in && x1 < g.Nx;
-                    val = B::template ld_cx<kStream>(rin, ok ? rowoff + (O)x0 * RB : B::OOB);
+                    val = B::template ld_cx<NTX>(rin, ok ? rowoff + (O)x0 * RB : B::OOB);
                     if (cvf)
                         val = cx<T>{ok && x0 >= xlo && x0 < xhi ? val.x - base : T(0),
                                     ok && x1 >= xlo && x1 < xhi ? val.y - base : T(0)};
                 } else {
                     const bool ok0 = n >= 0 && row_in && x0 >= xlo && x0 < xhi;
                     const bool ok1 = n >= 0 && row_in && x1 >= xlo && x1 < xhi;
-                    const T a0 = B::template ld_r<kStream>(rin, ok0 ? rowoff + (O)x0 * RB : B::OOB);
-                    const T a1 = B::template ld_r<kStream>(rin, ok1 ? rowoff + (O)x1 * RB : B::OOB);
+                    const T a0 = B::template ld_r<NTX>(rin, ok0 ? rowoff + (O)x0 * RB : B::OOB);
+                    const T a1 = B::template ld_r<NTX>(rin, ok1 ? rowoff + (O)x1 * RB : B::OOB);
                     val = cx<T>{ok0 ? a0 - base : T(0), ok1 ? a1 - base : T(0)};
                 }
                 v[b * Sh::R0 + r] = val;
@@ -208,7 +212,7 @@ xfwd_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
         for (int k = t; k <= L; k += C::TPF) {
             const cx<T> zk = lds.at(k == L ? 0 : k);
             const cx<T> zc = cconj(lds.at(k == 0 ? 0 : L - k));
-            B::template st_cx<kStream>(post(k, zk, zc), rwork, live ? dst + (O)k * CB : B::OOB);
+            B::template st_cx<NTX>(post(k, zk, zc), rwork, live ? dst + (O)k * CB : B::OOB);
         }
         // the next item's first LDS store happens after a barrier inside fft_regs
     }
@@ -256,6 +260,7 @@ xinv_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
     const long ngroups = (nrows + C::G - 1) / C::G;
     RowLds<T> lds{smem + gr * C::PITCH};
     constexpr unsigned RB = sizeof(T), CB = sizeof(cx<T>);
+    constexpr int NTX = C::POL;
     for (long item = blockIdx.x; item < ngroups * nfields; item += gridDim.x) {
         int f = (int)(item / ngroups);
         if constexpr (sizeof(T) == 4) {
@@ -360,10 +365,10 @@ xinv_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
                         if (upd) {
                             const cx<T> d = B::ld_cx(rdel, off);
                             o = cx<T>{upd_level(d.x, o.x, dec), upd_level(d.y, o.y, dec)};
-                            B::template st_cx<kStream>(cx<T>{T(0), T(0)}, rdel, off);
+                            B::template st_cx<NTX>(cx<T>{T(0), T(0)}, rdel, off);
                         }
                     }
-                    B::template st_cx<kStream>(o, rout, off);
+                    B::template st_cx<NTX>(o, rout, off);
                 } else {
                     const bool ok0 = n >= 0 && live && 2 * n < g.Nx;
                     const bool ok1 = n >= 0 && live && 2 * n + 1 < g.Nx;
@@ -378,12 +383,12 @@ xinv_kernel(const FieldBatch fb, GridDesc g, const cx<T>* __restrict__ twg, int 
                         if (upd) {
                             o0 = upd_level(B::ld_r(rdel, off0), o0, dec);
                             o1 = upd_level(B::ld_r(rdel, off1), o1, dec);
-                            B::template st_r<kStream>(T(0), rdel, off0);
-                            B::template st_r<kStream>(T(0), rdel, off1);
+                            B::template st_r<NTX>(T(0), rdel, off0);
+                            B::template st_r<NTX>(T(0), rdel, off1);
                         }
                     }
-                    B::template st_r<kStream>(o0, rout, off0);
-                    B::template st_r<kStream>(o1, rout, off1);
+                    B::template st_r<NTX>(o0, rout, off0);
+                    B::template st_r<NTX>(o1, rout, off1);
                 }
             }
         // the next item's first LDS store happens after a barrier inside fft_regs
@@ -413,7 +418,13 @@ __device__ __forceinline__ double2 kscale(double2 v, double k) { return double2{
 //              elements the forward left in registers (no LDS redistribution).
 // KS (fused mode): the kernel-spectrum format -- KS_REAL, KS_COMPLEX (R2C
 // layout, scaled by cd.scale), or KS_SEP (FP64 tables, K^ formed here).
-enum { KS_REAL = 0, KS_COMPLEX = 1, KS_SEP = 2 };
+// KS_ROWS (forward and inverse modes): rows that do not start on 128-byte lines
+// (standalone transforms on the R2C layout, px/2 + 1 elements a row).  A tile's
+// row segment then shares its lines with its neighbours whatever its width, so
+// nothing is non-temporal and every XCD takes a contiguous run of tiles: the
+// neighbours meet in one L2 (R2C and C2R
+// of 256x256x192: 231 -> 126 us, of 320^3 810 -> 328).
+enum { KS_REAL = 0, KS_COMPLEX = 1, KS_SEP = 2, KS_ROWS = 3 };
 
 // Which z-pass form an FP32 field with a separable table takes, from the
 // window radius R the table itself stores (tab[cd.sep_g]): 8, 12 or 16 -- the
@@ -478,13 +489,13 @@ __device__ __forceinline__ void col_tile(const FieldDesc& fd, const ColDesc& cd,
     // non-temporal loads only when a tile row spans whole 128-byte lines: a
     // narrower tile (long columns) shares each line with its neighbours, which
     // must still find it in the cache
-    constexpr int NTP = C::TC * (int)CB >= 128 ? kStream : kCacheDefault;
+    constexpr int NTP = C::TC * (int)CB >= 128 && KS != KS_ROWS ? kStream : kCacheDefault;
     // stores: non-temporal for whole 128-byte row segments; a narrower segment
     // is written back through the L2, where the tiles sharing its line merge.
     // (Choosing the L2 path at run time for the last, mostly empty tile of a
     // 1025-column row measured 10-30 % slower on the y forward and z FFT
     // passes; the direct z pass, one column per lane, gains from it.)
-    constexpr int NTS = C::TC * (int)CB >= 128 ? kStream : kCacheDefault;
+    constexpr int NTS = C::TC * (int)CB >= 128 && KS != KS_ROWS ? kStream : kCacheDefault;
     constexpr int NI = ShF::NB0 * ShF::R0;
     constexpr int NO = ShI::NBL * ShI::RL;
     constexpr int NK = ShF::NBL * ShF::RL;
@@ -700,8 +711,16 @@ __attribute__((amdgpu_waves_per_eu((col_waves_per_eu<T, MODE, ColCfg<T, Q, V, RS
 col_kernel(const FieldBatch fb, ColDesc cd, const cx<T>* __restrict__ twg) {
     using C = ColCfg<T, Q, V, RS>;
     unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
-    if constexpr (C::SH > 1)
+    if constexpr (KS == KS_ROWS) {
+        const unsigned per = (gridDim.x + 7u) / 8u;
+        const unsigned id = blockIdx.x % 8u * per + blockIdx.x / 8u;
+        bx = id % cd.grid_segs;
+        by = id / cd.grid_segs % cd.grid_planes;
+        bz = id / cd.grid_segs / cd.grid_planes;
+        if (bz >= cd.grid_fields) return;
+    } else if constexpr (C::SH > 1) {
         if (!col_coords<C>(cd, blockIdx.x, cd.grid_fields, bx, by, bz)) return;
+    }
     if constexpr (sizeof(T) == 4) {
         if (cd.records && dir_form((const char*)fb.f[bz].work + cd.rec_off)) return;  // not the FFT passes' field
     }

@@ -654,6 +654,7 @@ static int run_r2c(const Plan& p, const void* in, void* out, hipStream_t st) {
     y.mode = COL_FWD; y.rs = 1; y.nin = p.ny; y.nout = p.py; y.ncols = p.hx;
     y.rstride = p.ld; y.pstride = p.plane; y.scale = 1.0;
     y.work_bytes = cbytes;
+    y.off_lines = p.ld * 2 * p.prec % 128 != 0;
     e = launch_col<T>(p.py, fb, 1, y, p.nz, p.tw_y, st);
     if (e != hipSuccess) return hip_check(e, "r2c y launch");
     ColDesc z = y;
@@ -673,6 +674,7 @@ static int run_c2r(const Plan& p, void* in, void* out, hipStream_t st) {
     z.mode = COL_INV; z.rs = 1; z.nin = p.pz; z.nout = p.pz; z.ncols = p.hx;
     z.rstride = p.plane; z.pstride = p.ld; z.scale = 1.0;
     z.work_bytes = cbytes;
+    z.off_lines = p.ld * 2 * p.prec % 128 != 0;
     hipError_t e = launch_col<T>(p.pz, fb, 1, z, p.py, p.tw_z, st);
     if (e != hipSuccess) return hip_check(e, "c2r z launch");
     ColDesc y = z;

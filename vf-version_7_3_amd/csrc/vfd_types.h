@@ -76,6 +76,7 @@ struct ColDesc {
     unsigned grid_ids;  // ids of a 1-D launch (grid_segs = tiles per row where tiles are not narrow)
     int records;        // Records: fields of the direct form are left out
     unsigned long rec_off;
+    int off_lines;      // rows do not start on 128-byte lines (KS_ROWS)
     int sep_g;          // separable: table offset (elements) of [R | g_0 .. g_kZDirectMaxR]
     int fold;           // rs = 2 with output rows past P/2 (FP32 inverse-only, fold_supported)
 };
