@@ -31,18 +31,12 @@ template <int Q, int V, bool FWD>
 hipError_t zr_go(const FieldBatch& fields, int nfields, const XlDesc& d, const void* tw, hipStream_t st) {
     using C = ColCfg<float, Q, V, 1>;
     XlDesc g = d;
-    if constexpr (C::SH > 1) {
-        g.grid_segs = (unsigned)((d.ncolp + C::TC_LINE - 1) / C::TC_LINE);
-        g.grid_fields = (unsigned)nfields;
-        const unsigned long groups = (unsigned long)g.grid_segs * nfields;
-        const unsigned long ids = (groups + 7) / 8 * 8 * C::SH;
-        if (ids > 0x7fffffffu) return hipErrorInvalidConfiguration;
-        hipLaunchKernelGGL((zr_kernel<float, Q, V, FWD>), dim3((unsigned)ids), dim3(C::NT), 0, st, fields, g,
-                           (const float2*)tw);
-    } else {
-        dim3 grid((unsigned)((d.ncolp + C::TC - 1) / C::TC), (unsigned)nfields);
-        hipLaunchKernelGGL((zr_kernel<float, Q, V, FWD>), grid, dim3(C::NT), 0, st, fields, g, (const float2*)tw);
-    }
+    g.grid_segs = (unsigned)((d.ncolp + C::TC - 1) / C::TC);
+    g.grid_fields = (unsigned)nfields;
+    const unsigned long ids = ((unsigned long)g.grid_segs * nfields + 7) / 8 * 8;
+    if (ids > 0x7fffffffu) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL((zr_kernel<float, Q, V, FWD>), dim3((unsigned)ids), dim3(C::NT), 0, st, fields, g,
+                       (const float2*)tw);
     return hipGetLastError();
 }
 

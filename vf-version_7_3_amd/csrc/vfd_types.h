@@ -96,7 +96,7 @@ struct XlDesc {
     int pad_mode;        // PadMode
     double scale;        // applied to K^ products (1 / (px py pz))
     unsigned long in_bytes, work_bytes, kspec_bytes, out_bytes;  // per-field array sizes
-    // grouped 1-D launch of narrow tiles (set by the launcher)
+    // 1-D launch of the z passes (set by the launcher)
     unsigned grid_fields, grid_segs;
 };
 

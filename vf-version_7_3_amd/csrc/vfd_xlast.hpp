@@ -45,15 +45,20 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
     constexpr unsigned CB = sizeof(cx<T>), RB = sizeof(T);
     __shared__ cx<T> smem[C::TC * Q];
     __shared__ cx<T> tw[Q];
-    unsigned bx = blockIdx.x, bf = blockIdx.y;
-    if constexpr (C::SH > 1) {
-        const unsigned lin = blockIdx.x;
-        const unsigned grp = (lin / (8u * C::SH)) * 8u + lin % 8u;
-        bx = (grp % d.grid_segs) * C::SH + (lin / 8u) % C::SH;
-        bf = grp / d.grid_segs;
-        // whole-block exits, before any barrier: padding ids, tiles past the end
-        if (bf >= d.grid_fields || (long)bx * C::TC >= d.ncolp) return;
-    }
+    // Every XCD takes a contiguous run of tiles.  A data row (440 bytes in the
+    // production box) rarely starts on a 128-byte line, and neither does a tile's
+    // segment of it, so neighbouring tiles share lines at every plane: they meet
+    // in one L2, and nothing is non-temporal.  Dealt out over the XCDs in groups
+    // of a line, z R2C fetched 1.15 GB for 0.61 and z C2R wrote 1.06 GB for 0.61.
+    // 1006x1390x110 in 1152x1536x256: 664 -> 620 us and 557 -> 522; 301x203x75 in
+    // 384x256x128: 22.7 -> 16.3 and 24.7 -> 18.4.  What is left is the memory's:
+    // the same loads and stores without the transforms take 500 and 404 us.
+    // (Rows tiled by themselves, so that no tile crosses one: 630 and 517, and a
+    // quarter of the tiles padding at 75 columns.  Tiles of 8 pairs for the long
+    // columns, stages exchanged one component at a time: 880 and 620.)
+    const unsigned id = blockIdx.x % 8u * (gridDim.x / 8u) + blockIdx.x / 8u;
+    const unsigned bx = id % d.grid_segs, bf = id / d.grid_segs;
+    if (bf >= d.grid_fields) return;  // whole-block exit, before any barrier: padding ids
     const FieldDesc& fd = fb.f[bf];
     const int c = threadIdx.x % C::TC;
     const int t = threadIdx.x / C::TC;
@@ -68,13 +73,6 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
     const O dcol = (O)((long)y * d.nx + x0) * RB;   // data (z, y, x0) = dcol + z * dstep
     const O dstep = (O)((long)d.ny * d.nx) * RB;
     const bool vec = d.nx % 2 == 0;                  // x0, x0+1 in one 8-byte word
-    // non-temporal accesses where a tile row spans whole 128-byte lines (loads)
-    // or 64-byte segments (stores); narrower rows share lines with neighbouring
-    // tiles, which must find them in (or merge them through) the L2
-    constexpr int NTP = C::TC * (int)RB * 2 >= 128 ? kStream : kCacheDefault;   // field rows
-    constexpr int NTW = C::TC * (int)CB * 2 >= 128 ? kStream : kCacheDefault;   // work rows
-    constexpr int NTSF = C::TC * (int)RB * 2 >= 128 ? kStream : kCacheDefault;   // field stores
-    constexpr int NTSW = C::TC * (int)CB * 2 >= 128 ? kStream : kCacheDefault;   // work stores
     cx<T> v[Sh::E];
 
     if constexpr (FWD) {
@@ -98,11 +96,11 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                 if (vec) {
                     // the pair in one load (both voxels are in the row); the
                     // constant pad's faces are cut afterwards
-                    val = B::template ld_cx<NTP>(rin, zin && (in0 || in1) ? off : B::OOB);
+                    val = B::template ld_cx<kCacheDefault>(rin, zin && (in0 || in1) ? off : B::OOB);
                     if (cvf) val = cx<T>{zin && in0 ? val.x - base : T(0), zin && in1 ? val.y - base : T(0)};
                 } else {
-                    const T a0 = B::template ld_r<NTP>(rin, zin && in0 ? off : B::OOB);
-                    const T a1 = B::template ld_r<NTP>(rin, zin && in1 ? off + RB : B::OOB);
+                    const T a0 = B::template ld_r<kCacheDefault>(rin, zin && in0 ? off : B::OOB);
+                    const T a1 = B::template ld_r<kCacheDefault>(rin, zin && in1 ? off + RB : B::OOB);
                     val = cx<T>{zin && in0 ? a0 - base : T(0), zin && in1 ? a1 - base : T(0)};
                 }
                 v[b * Sh::R0 + r] = val;
@@ -129,7 +127,7 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                 const cx<T> cc = cconj(lds.at(ok && k > 0 ? Q - k : 0));
                 const cx<T> s = cscale(cadd(ck, cc), T(0.5));
                 const cx<T> dd = cscale(csub(ck, cc), T(0.5));
-                B::template st_cx2<NTSW>(s, cx<T>{dd.y, -dd.x}, rwork, ok ? wcol + (O)k * wstep : B::OOB);
+                B::template st_cx2<kCacheDefault>(s, cx<T>{dd.y, -dd.x}, rwork, ok ? wcol + (O)k * wstep : B::OOB);
             }
     } else {
         // The half spectrum (rows 0..Q/2) of the tile's column pairs is read
@@ -147,7 +145,7 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int m = t + i * C::TPF;
-            B::template ld_cx2<NTW>(rwork, m < HZ && live ? wcol + (O)m * wstep : B::OOB, ha[i], hb[i]);
+            B::template ld_cx2<kCacheDefault>(rwork, m < HZ && live ? wcol + (O)m * wstep : B::OOB, ha[i], hb[i]);
         }
         stage_table_unrolled<Q, C::NT>(tw, twg, Q);
 #pragma unroll
@@ -234,10 +232,10 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                             const cx<T> dl = B::ld_cx(rdel, ok ? off : B::OOB);
                             o0 = upd_level(dl.x, o0, dec);
                             o1 = upd_level(dl.y, o1, dec);
-                            B::template st_cx<NTSF>(cx<T>{T(0), T(0)}, rdel, ok ? off : B::OOB);
+                            B::template st_cx<kCacheDefault>(cx<T>{T(0), T(0)}, rdel, ok ? off : B::OOB);
                         }
                     }
-                    B::template st_cx<NTSF>(cx<T>{o0, o1}, rout, ok ? off : B::OOB);
+                    B::template st_cx<kCacheDefault>(cx<T>{o0, o1}, rout, ok ? off : B::OOB);
                 } else {
                     const O off0 = ok ? off : B::OOB;
                     const O off1 = ok && has1 ? off + RB : B::OOB;
@@ -245,12 +243,12 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                         if (upd) {
                             o0 = upd_level(B::ld_r(rdel, off0), o0, dec);
                             o1 = upd_level(B::ld_r(rdel, off1), o1, dec);
-                            B::template st_r<NTSF>(T(0), rdel, off0);
-                            B::template st_r<NTSF>(T(0), rdel, off1);
+                            B::template st_r<kCacheDefault>(T(0), rdel, off0);
+                            B::template st_r<kCacheDefault>(T(0), rdel, off1);
                         }
                     }
-                    B::template st_r<NTSF>(o0, rout, off0);
-                    B::template st_r<NTSF>(o1, rout, off1);
+                    B::template st_r<kCacheDefault>(o0, rout, off0);
+                    B::template st_r<kCacheDefault>(o1, rout, off1);
                 }
             }
     }
