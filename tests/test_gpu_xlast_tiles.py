@@ -18,6 +18,7 @@ REL_F32 = 1e-5
     ((3, 3, 3), (1536, 32, 32), 100, 0, 0.0),       # mostly padding, one tile a field
     ((40, 33, 25), (64, 64, 32), 3, 20, 0.2),       # short columns
     ((20, 17, 33), (32, 32, 64), 100, 0, 0.0),
+    ((201, 100, 71), (256, 128, 128), 3, 60, 0.2),  # more than the L2s hold: no rows streamed
 ])
 def test_z_tiles_of_a_batch_every_schedule(vfd, orc, monkeypatch, shape, box, pad, epi, base):
     """FP32 tolerance of the x-last order's other tests."""

@@ -27,6 +27,17 @@ int cu_count() {
     return ncu;
 }
 
+// Whether the z passes' whole-line rows are non-temporal: where the launch's
+// fields and work arrays fit in the L2s together (8 x 4 MB) the passes between
+// gain more from what they leave there than the z passes lose on shared lines.
+// Ticks, non-temporal against default: 142x100x60 in 256x128x128 (11 MB) 37.8 against
+// 40.5 us; 200x100x150 in 256x128x384 (32 MB) 72.7 against 74.4; 500x101x73 in
+// 768x128x192 (37 MB) 94.5 against 89.6; 301x203x75 in 384x256x128, 1 field (49 MB)
+// 82 against 77, 4 fields 323 against 267.
+bool zr_streams(int nfields, const XlDesc& d) {
+    return (unsigned long)nfields * (d.in_bytes + d.work_bytes) <= (32ul << 20);
+}
+
 template <int Q, int V, bool FWD>
 hipError_t zr_go(const FieldBatch& fields, int nfields, const XlDesc& d, const void* tw, hipStream_t st) {
     using C = ColCfg<float, Q, V, 1>;
@@ -35,8 +46,13 @@ hipError_t zr_go(const FieldBatch& fields, int nfields, const XlDesc& d, const v
     g.grid_fields = (unsigned)nfields;
     const unsigned long ids = ((unsigned long)g.grid_segs * nfields + 7) / 8 * 8;
     if (ids > 0x7fffffffu) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((zr_kernel<float, Q, V, FWD>), dim3((unsigned)ids), dim3(C::NT), 0, st, fields, g,
-                       (const float2*)tw);
+    constexpr bool WIDE = C::TC * 16 >= 128;  // a tile's work row is a line: there are rows to stream
+    if (WIDE && zr_streams(nfields, d))
+        hipLaunchKernelGGL((zr_kernel<float, Q, V, FWD, WIDE>), dim3((unsigned)ids), dim3(C::NT), 0, st, fields, g,
+                           (const float2*)tw);
+    else
+        hipLaunchKernelGGL((zr_kernel<float, Q, V, FWD, false>), dim3((unsigned)ids), dim3(C::NT), 0, st, fields, g,
+                           (const float2*)tw);
     return hipGetLastError();
 }
 

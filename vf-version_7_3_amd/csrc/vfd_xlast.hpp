@@ -35,7 +35,8 @@ namespace vfd {
 // unnormalized inverse FFT, a = Re c, b = Im c cropped to nz.
 // A work-group owns TC column pairs; narrow tiles use the grouped 1-D launch
 // of col_kernel (the SH tiles sharing a 128-byte input segment run on one XCD).
-template <typename T, int Q, int V, bool FWD>
+// NT: rows of whole 128-byte lines non-temporal (zr_streams), else nothing is.
+template <typename T, int Q, int V, bool FWD, bool NT>
 __global__ void __launch_bounds__((ColCfg<T, Q, V, 1>::NT))
 zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
     using C = ColCfg<T, Q, V, 1>;
@@ -48,7 +49,7 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
     // Every XCD takes a contiguous run of tiles.  A data row (440 bytes in the
     // production box) rarely starts on a 128-byte line, and neither does a tile's
     // segment of it, so neighbouring tiles share lines at every plane: they meet
-    // in one L2, and nothing is non-temporal.  Dealt out over the XCDs in groups
+    // in one L2 (and nothing is non-temporal, but see zr_streams).  Dealt out over the XCDs in groups
     // of a line, z R2C fetched 1.15 GB for 0.61 and z C2R wrote 1.06 GB for 0.61.
     // 1006x1390x110 in 1152x1536x256: 664 -> 620 us and 557 -> 522; 301x203x75 in
     // 384x256x128: 22.7 -> 16.3 and 24.7 -> 18.4.  What is left is the memory's:
@@ -73,6 +74,8 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
     const O dcol = (O)((long)y * d.nx + x0) * RB;   // data (z, y, x0) = dcol + z * dstep
     const O dstep = (O)((long)d.ny * d.nx) * RB;
     const bool vec = d.nx % 2 == 0;                  // x0, x0+1 in one 8-byte word
+    constexpr int PF = NT && C::TC * (int)RB * 2 >= 128 ? kStream : kCacheDefault;  // field rows
+    constexpr int PW = NT && C::TC * (int)CB * 2 >= 128 ? kStream : kCacheDefault;  // work rows
     cx<T> v[Sh::E];
 
     if constexpr (FWD) {
@@ -96,11 +99,11 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                 if (vec) {
                     // the pair in one load (both voxels are in the row); the
                     // constant pad's faces are cut afterwards
-                    val = B::template ld_cx<kCacheDefault>(rin, zin && (in0 || in1) ? off : B::OOB);
+                    val = B::template ld_cx<PF>(rin, zin && (in0 || in1) ? off : B::OOB);
                     if (cvf) val = cx<T>{zin && in0 ? val.x - base : T(0), zin && in1 ? val.y - base : T(0)};
                 } else {
-                    const T a0 = B::template ld_r<kCacheDefault>(rin, zin && in0 ? off : B::OOB);
-                    const T a1 = B::template ld_r<kCacheDefault>(rin, zin && in1 ? off + RB : B::OOB);
+                    const T a0 = B::template ld_r<PF>(rin, zin && in0 ? off : B::OOB);
+                    const T a1 = B::template ld_r<PF>(rin, zin && in1 ? off + RB : B::OOB);
                     val = cx<T>{zin && in0 ? a0 - base : T(0), zin && in1 ? a1 - base : T(0)};
                 }
                 v[b * Sh::R0 + r] = val;
@@ -127,7 +130,7 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                 const cx<T> cc = cconj(lds.at(ok && k > 0 ? Q - k : 0));
                 const cx<T> s = cscale(cadd(ck, cc), T(0.5));
                 const cx<T> dd = cscale(csub(ck, cc), T(0.5));
-                B::template st_cx2<kCacheDefault>(s, cx<T>{dd.y, -dd.x}, rwork, ok ? wcol + (O)k * wstep : B::OOB);
+                B::template st_cx2<PW>(s, cx<T>{dd.y, -dd.x}, rwork, ok ? wcol + (O)k * wstep : B::OOB);
             }
     } else {
         // The half spectrum (rows 0..Q/2) of the tile's column pairs is read
@@ -145,7 +148,7 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int m = t + i * C::TPF;
-            B::template ld_cx2<kCacheDefault>(rwork, m < HZ && live ? wcol + (O)m * wstep : B::OOB, ha[i], hb[i]);
+            B::template ld_cx2<PW>(rwork, m < HZ && live ? wcol + (O)m * wstep : B::OOB, ha[i], hb[i]);
         }
         stage_table_unrolled<Q, C::NT>(tw, twg, Q);
 #pragma unroll
@@ -232,10 +235,10 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                             const cx<T> dl = B::ld_cx(rdel, ok ? off : B::OOB);
                             o0 = upd_level(dl.x, o0, dec);
                             o1 = upd_level(dl.y, o1, dec);
-                            B::template st_cx<kCacheDefault>(cx<T>{T(0), T(0)}, rdel, ok ? off : B::OOB);
+                            B::template st_cx<PF>(cx<T>{T(0), T(0)}, rdel, ok ? off : B::OOB);
                         }
                     }
-                    B::template st_cx<kCacheDefault>(cx<T>{o0, o1}, rout, ok ? off : B::OOB);
+                    B::template st_cx<PF>(cx<T>{o0, o1}, rout, ok ? off : B::OOB);
                 } else {
                     const O off0 = ok ? off : B::OOB;
                     const O off1 = ok && has1 ? off + RB : B::OOB;
@@ -243,12 +246,12 @@ zr_kernel(const FieldBatch fb, XlDesc d, const cx<T>* __restrict__ twg) {
                         if (upd) {
                             o0 = upd_level(B::ld_r(rdel, off0), o0, dec);
                             o1 = upd_level(B::ld_r(rdel, off1), o1, dec);
-                            B::template st_r<kCacheDefault>(T(0), rdel, off0);
-                            B::template st_r<kCacheDefault>(T(0), rdel, off1);
+                            B::template st_r<PF>(T(0), rdel, off0);
+                            B::template st_r<PF>(T(0), rdel, off1);
                         }
                     }
-                    B::template st_r<kCacheDefault>(o0, rout, off0);
-                    B::template st_r<kCacheDefault>(o1, rout, off1);
+                    B::template st_r<PF>(o0, rout, off0);
+                    B::template st_r<PF>(o1, rout, off1);
                 }
             }
     }
