@@ -27,7 +27,7 @@ template <typename T>
 hipError_t launch_col(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
                       const void* tw, hipStream_t st, int variant = 0);
 
-// the FP32 column pass of a batch with RECORDS_FEW: launch_col calls it
+// the FP32 column pass of a batch with records: launch_col calls it
 hipError_t launch_col_rec(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
                           const void* tw, hipStream_t st, int variant);
 

@@ -160,22 +160,6 @@ static bool col_ids(ColDesc& g, int nfields, long nplanes) {
     return ids <= 0x7ffffffful;
 }
 
-#ifdef VFD_COLREC_TU
-// the launches of batches with records (FP32): col_rec_kernel
-template <typename T, int Q, int MODE, int RS, int V, int KS = KS_REAL, bool FOLD = false>
-static hipError_t col_go(const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
-                         const void* tw, hipStream_t st) {
-    using C = ColCfg<T, Q, V, RS>;
-    ColDesc g = cd;
-    if (!col_ids<C>(g, nfields, nplanes)) return hipErrorInvalidConfiguration;
-    // as many work-groups as the card holds, at most one per tile
-    static const int per_cu = blocks_per_cu(col_rec_kernel<Q, MODE, RS, V, KS, FOLD>, C::NT);
-    const unsigned cap = (unsigned)(num_cus() * per_cu);
-    hipLaunchKernelGGL((col_rec_kernel<Q, MODE, RS, V, KS, FOLD>), dim3(g.grid_ids < cap ? g.grid_ids : cap), dim3(C::NT), 0,
-                       st, fields, g, (const cx<T>*)tw);
-    return hipGetLastError();
-}
-#else
 template <typename T, int Q, int MODE, int RS, int V, int KS = KS_REAL, bool FOLD = false>
 static hipError_t col_go(const FieldBatch& fields, int nfields, const ColDesc& cd, long nplanes,
                          const void* tw, hipStream_t st) {
@@ -183,16 +167,29 @@ static hipError_t col_go(const FieldBatch& fields, int nfields, const ColDesc& c
     ColDesc g = cd;
     if (!col_ids<C>(g, nfields, nplanes)) return hipErrorInvalidConfiguration;
     dim3 grid = C::SH > 1 ? dim3(g.grid_ids) : dim3(g.grid_segs, (unsigned)nplanes, (unsigned)nfields);
+#ifdef VFD_COLREC_TU
+    constexpr bool REC = true;
+    if (cd.records == RECORDS_FEW) {
+        // as many work-groups as the card holds, at most one per tile
+        static const int per_cu = blocks_per_cu(col_rec_kernel<Q, MODE, RS, V, KS, FOLD>, C::NT);
+        const unsigned cap = (unsigned)(num_cus() * per_cu);
+        hipLaunchKernelGGL((col_rec_kernel<Q, MODE, RS, V, KS, FOLD>), dim3(g.grid_ids < cap ? g.grid_ids : cap),
+                           dim3(C::NT), 0, st, fields, g, (const cx<T>*)tw);
+        return hipGetLastError();
+    }
+#else
+    constexpr bool REC = false;
     if constexpr (KS == KS_ROWS) {  // every tile by itself, whole rounds of XCDs
         g.grid_segs = (unsigned)((cd.ncols + C::TC - 1) / C::TC);
         const unsigned long ids = ((unsigned long)g.grid_segs * nplanes * nfields + 7) / 8 * 8;
         if (ids > 0x7fffffffu) return hipErrorInvalidConfiguration;
         grid = dim3((unsigned)ids);
     }
-    hipLaunchKernelGGL((col_kernel<T, Q, MODE, RS, V, KS, FOLD>), grid, dim3(C::NT), 0, st, fields, g, (const cx<T>*)tw);
+#endif
+    hipLaunchKernelGGL((col_kernel<T, Q, MODE, RS, V, KS, FOLD, REC>), grid, dim3(C::NT), 0, st, fields, g,
+                       (const cx<T>*)tw);
     return hipGetLastError();
 }
-#endif
 
 // fused pass: the spectrum format picks the instantiation
 template <typename T, int Q, int RS, int V>
@@ -257,7 +254,7 @@ template <>
 hipError_t launch_col<VFD_REAL>(int Q, const FieldBatch& fields, int nfields, const ColDesc& cd,
                                 long nplanes, const void* tw, hipStream_t st, int variant) {
     if constexpr (sizeof(VFD_REAL) == 4) {
-        if (cd.records == RECORDS_FEW) return launch_col_rec(Q, fields, nfields, cd, nplanes, tw, st, variant);
+        if (cd.records) return launch_col_rec(Q, fields, nfields, cd, nplanes, tw, st, variant);
     }
 #endif
     constexpr bool kVariants = sizeof(VFD_REAL) == 4;  // FP64 has one schedule
