@@ -8,10 +8,12 @@ times exp(-lambda dt) (lambda ~ U[0.001,0.05]); lognormal(-2,1) background
 plus 50 point sources of amplitude U[1,100].  Inputs are synthetic and
 generated on the device; kernel spectra are precomputed and resident.
 
-A step = one tick of all fields (5 HBM passes per field, all fields batched
-into each launch; the z pass is four launches: the direct form for window
-radius bounds 8, 12, 16 and the FFT form, each acting on its own fields).  W
-untimed warmup steps, then K timed steps bracketed by torch.cuda.synchronize().
+A step = one tick of all fields, all fields batched into each launch.  Separable
+windows up to radius 31 (every field of the default workload) take the direct
+form: 2 HBM passes, x-y and z, which run in the first and the last launch.
+Other fields take the FFT form: 5 passes, of which the z pass is four launches
+(direct in z for window radius bounds 8, 12, 16, and FFT), each acting on its
+own fields.  W untimed warmup steps, then K timed steps bracketed by torch.cuda.synchronize().
 Per-kernel durations come from HIP events recorded between the launches on the
 launch stream over the timed region; roofline.kernel is the single kernel with
 the largest average duration, roofline.step_frac the whole step.  copy_gbs is
@@ -509,6 +511,7 @@ def bench_ensemble(args):
     """Batched (graph) vs plain per-field ticks over uneven resident runs."""
     import numpy as np
     import torch
+    import vfd
     import vfd.engine as ve
     rng = np.random.default_rng(args.seed)
     nf = args.fields
@@ -551,11 +554,9 @@ def bench_ensemble(args):
     if "reference" in forms:
         t["reference"] = reference_flow_tick(picks, nf, args.seed)
     counts = {f"{s[2]}x{s[1]}x{s[0]}": int((picks == i).sum()) for i, s in enumerate(ENSEMBLE_GRIDS)}
-    bytes_tick = 0.0
-    for i, s in enumerate(ENSEMBLE_GRIDS):
-        import vfd
-        p = vfd.Plan(s, kspec_format=vfd.KSPEC_SEPARABLE)
-        bytes_tick += p.info.bytes_per_field_tick * nf * counts[f"{s[2]}x{s[1]}x{s[0]}"]
+    # every window is within radius 19, the direct form: a field is read and
+    # written by the x-y and by the z pass
+    bytes_tick = sum(16.0 * s[0] * s[1] * s[2] * nf * counts[f"{s[2]}x{s[1]}x{s[0]}"] for s in ENSEMBLE_GRIDS)
     head = forms[0]
     out = _header(args, f"voxel-updates/s, ensemble tick (64 uneven runs x 8 fields), {head} form", vox / t[head],
                   "voxel-updates/s", t[head] * 1e3,
@@ -804,7 +805,10 @@ def mix_bandwidth(vfd, torch, stream, nbytes=1 << 30, reps=7):
 
 # read:write mix of each launch of the step (x-first order)
 LAUNCH_MIX = {"xfwd": "r1w2", "yfwd": "r1w2", "z_direct8": "r1w1", "z_direct12": "r1w1", "z_direct16": "r1w1",
-              "z_fft": "r1w1", "yinv": "r2w1", "xinv": "r2w1"}
+              "z_fft": "r1w1", "yinv": "r2w1", "xinv": "r2w1", "dir_xy": "r1w1", "dir_z": "r1w1"}
+
+# largest window radius of the direct form (every axis' window within it)
+DIRECT_MAX_R = 31
 
 
 def fft_z_step(vfd, torch, np, shape, fields, params, model_bytes, stream, warmup, steps):
@@ -973,18 +977,29 @@ def main():
     ms_per_step = wall * 1e3 / K
     vox = float(nz * ny * nx) * nf
     value = vox * K / wall
-    # fields per launch: the z launches act on the fields of their own form
-    # (window radius R = ceil(6 sigma) <= 8, <= 12, <= 16 direct; beyond, FFT)
+    # fields per launch: window radius R = ceil(6 sigma) <= 31 takes the direct
+    # form (a field read and written by x-y in the first launch and by z in the
+    # last); the z launches act on the other fields of their own form
+    # (R <= 8, <= 12, <= 16 direct in z; beyond, FFT)
     radii = [int(np.ceil(6.0 * np.sqrt(s2))) for s2, _ in params]
     if kfmt == vfd.KSPEC_SEPARABLE:
-        forms = [0 if r <= 8 else 1 if r <= 12 else 2 if r <= 16 else 3 for r in radii]
+        rest = [r for r in radii if r > DIRECT_MAX_R or r > min(shape)]
+        forms = [0 if r <= 8 else 1 if r <= 12 else 2 if r <= 16 else 3 for r in rest]
     else:
+        rest = radii
         forms = [3] * nf
-    kern_fields = [nf, nf] + [forms.count(i) for i in range(4)] + [nf, nf]
+    nfft, ndir = len(rest), nf - len(rest)
+    kern_fields = [nfft, nfft] + [forms.count(i) for i in range(4)] + [nfft, nfft]
     kern_bytes = [plan.pass_bytes(p) * kern_fields[i] for i, (_, p) in enumerate(launches)]
+    if ndir:
+        field_rw = 8.0 * nx * ny * nz  # one FP32 field read and written
+        for i, name in ((0, "dir_xy"), (nl - 1, "dir_z")):
+            kern_bytes[i] += field_rw * ndir
+            kern_fields[i] = nf
+            launches[i] = (name if nfft == 0 else launches[i][0], launches[i][1])
     kern_gbs = [b / (t * 1e-3) / 1e9 if t > 0 else 0.0 for b, t in zip(kern_bytes, kern_ms)]
     dom = int(np.argmax(kern_ms))
-    step_bytes = plan.info.bytes_per_field_tick * nf
+    step_bytes = sum(kern_bytes)
     mean_step_ms = float(np.mean(step_ms))
     copy_gbs = copy_bandwidth(vfd, torch, stream)
     mix_gbs = mix_bandwidth(vfd, torch, stream)
@@ -1036,9 +1051,10 @@ def main():
             "kernels_frac_of_mix": {n: (g / mix_gbs[LAUNCH_MIX[n]] if g > 0 else None)
                                     for (n, _), g in zip(launches, kern_gbs)},
             # the five-pass byte model with a streamed real K^ (8N + 32 A1 + 32 A2 + 4 A3):
-            # counts 4 A3 per field that the separable spectrum never reads
+            # counts 4 A3 per field that the separable spectrum never reads; a step
+            # with fields of the direct form does not move these bytes at all
             "model_bytes_per_step": model_bytes,
-            "model_frac": model_bytes / (mean_step_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
+            "model_frac": None if ndir else model_bytes / (mean_step_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
         },
     }
     if fft_z is not None:
