@@ -161,7 +161,19 @@ constexpr int dir_r4(int rb) { return (rb + 3) / 4 * 4; }
 constexpr int dir_batch(int tx) { return kDirThreads * kDirOut / tx; }
 constexpr int dir_ring_rows(int tx, int rb) { return dir_batch(tx) + 2 * dir_r4(rb); }
 
-template <int RB> struct DirTaps {
+// The radius bounds that form their outputs in pairs (DirTaps<RB, true>): where
+// the pass is bound by its vector instructions.  x-y of 4 fields 512x512x128, one
+// by one against in pairs: R = 6 235 / 233 us (the memory's time either way), 8
+// 243 / 237, 12 295 / 262, 16 351 / 312, 20 450 / 404, 24 504 / 462, 31 615 / 573;
+// z 212 / 211 at 12, 250 / 236 at 20, 310 / 281 at 31; a tick of 8 fields
+// 1024x512x128 (R 6 - 19) 1950 -> 1811.  Windows narrower than 8 fall off too
+// fast from tap to tap for their differences to be small: beside a value 1000
+// times its own, an output at R = 1 lost 1e-5 of itself.  (A wide window with
+// such a step errs by 1e-7 of the step times the largest value, as the FFT
+// passes do.)  Against 64 bits a tick's rel-L2 is 6.2e-8 either way.
+constexpr bool dir_pairs(int rb) { return rb >= 8; }
+
+template <int RB, bool PAIRS = dir_pairs(RB)> struct DirTaps {
     float t[RB + 1];
     __device__ __forceinline__ void load(const DirAxis* a) {
 #pragma unroll
@@ -174,7 +186,7 @@ template <int RB> struct DirTaps {
 // so the taps first grow to the centre (lo) and then shrink (hi); one running
 // sum would round every term after the centre at the full magnitude of the
 // result (rel-L2 of a tick 1.0e-7 instead of 0.7e-7).
-struct DirSums {
+template <bool PAIRS> struct DirSums {
     float lo[kDirOut], hi[kDirOut];
     __device__ __forceinline__ DirSums() {
 #pragma unroll
@@ -185,9 +197,13 @@ struct DirSums {
 #pragma unroll
         for (int v = 0; v < kDirOut; ++v) asm volatile("" : "+v"(lo[v]), "+v"(hi[v]));
     }
-    // input element idx (0 .. 7 + 2 RB4) of the run that starts RB4 before the
-    // first of the 8 outputs
-    template <int RB> __device__ __forceinline__ void add(const DirTaps<RB>& tp, float in, int idx) {
+    // input elements idx, idx + 1 (0 .. 7 + 2 RB4) of the run that starts RB4
+    // before the first of the 8 outputs
+    template <int RB> __device__ __forceinline__ void add(const DirTaps<RB>& tp, float i0, float i1, int idx) {
+        add1<RB>(tp, i0, idx);
+        add1<RB>(tp, i1, idx + 1);
+    }
+    template <int RB> __device__ __forceinline__ void add1(const DirTaps<RB>& tp, float in, int idx) {
         constexpr int RB4 = dir_r4(RB);
 #pragma unroll
         for (int v = 0; v < kDirOut; ++v) {
@@ -199,9 +215,74 @@ struct DirSums {
     }
 };
 
+// Outputs are formed in pairs from pairs of inputs (e, o), o one after e: with
+// h the window,
+//   y[0] = sum h[2i] (e + o)[i] + sum (h[2i+1] - h[2i]) o[i]
+//   y[1] = sum h[2i] (e + o)[i] + sum (h[2i-1] - h[2i]) e[i],
+// of which the first sum is shared: 3 R + 2 products a pair and one sum an input
+// pair instead of 4 R + 2 products.  The differences of an even window are two
+// lists, of which the second sum runs one forwards and the third backwards.
+template <int RB> struct DirTaps<RB, true> {
+    static constexpr int NE = RB / 2 + 1, NB = (RB + 1) / 2;
+    float e[NE];      // h[2i]
+    float up[NE];     // h[2i+1] - h[2i]
+    float dn[NB + 1]; // h[2i-1] - h[2i], i >= 1
+    __device__ __forceinline__ void load(const DirAxis* a) {
+        auto uni = [](float v) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+        };
+        auto h = [&](int j) { return j <= RB ? a->tap[j] : 0.0f; };
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            e[i] = uni(h(2 * i));
+            up[i] = uni(h(2 * i + 1) - h(2 * i));
+        }
+        dn[0] = 0.0f;
+#pragma unroll
+        for (int i = 1; i <= NB; ++i) dn[i] = uni(h(2 * i - 1) - h(2 * i));
+    }
+};
+
+// the outputs as 4 pairs: the shared sum in two parts, and the differences' sums
+template <> struct DirSums<true> {
+    float lo[kDirOut / 2], hi[kDirOut / 2], d[kDirOut];
+    __device__ __forceinline__ DirSums() {
+#pragma unroll
+        for (int m = 0; m < kDirOut / 2; ++m) lo[m] = hi[m] = d[2 * m] = d[2 * m + 1] = 0.0f;
+    }
+    __device__ __forceinline__ float operator[](int v) const { return lo[v / 2] + hi[v / 2] + d[v]; }
+    __device__ __forceinline__ void pin() {
+#pragma unroll
+        for (int m = 0; m < kDirOut / 2; ++m)
+            asm volatile("" : "+v"(lo[m]), "+v"(hi[m]), "+v"(d[2 * m]), "+v"(d[2 * m + 1]));
+    }
+    // input elements idx, idx + 1 (idx even, 0 .. 6 + 2 RB4) of the run that
+    // starts RB4 before the first of the 8 outputs
+    template <int RB> __device__ __forceinline__ void add(const DirTaps<RB>& tp, float ev, float od, int idx) {
+        constexpr int RB4 = dir_r4(RB);
+        const int j = idx / 2 - RB4 / 2;
+        const float s = ev + od;
+#pragma unroll
+        for (int m = 0; m < kDirOut / 2; ++m) {
+            const int i = j - m, n = i < 0 ? -i : i;
+            if (2 * n <= RB) {
+                float& a = i <= 0 ? lo[m] : hi[m];
+                a = fmaf(tp.e[n], s, a);
+                float& u = i >= 0 ? d[2 * m] : d[2 * m + 1];
+                u = fmaf(tp.up[n], i >= 0 ? od : ev, u);
+                if (i == 0) d[2 * m + 1] = fmaf(tp.up[0], ev, d[2 * m + 1]);
+            }
+            if (n > 0 && 2 * n - 1 <= RB) {
+                float& u = i < 0 ? d[2 * m] : d[2 * m + 1];
+                u = fmaf(tp.dn[n], i < 0 ? od : ev, u);
+            }
+        }
+    }
+};
+
 // 8 outputs of one ring column: `start` is the ring row of the first input
 template <int TX, int RB>
-__device__ __forceinline__ void dir_ring_conv(DirSums& acc, const DirTaps<RB>& tp, const float* ring, int start,
+__device__ __forceinline__ void dir_ring_conv(DirSums<dir_pairs(RB)>& acc, const DirTaps<RB>& tp, const float* ring, int start,
                                               int col) {
     constexpr int RB4 = dir_r4(RB), RS = dir_ring_rows(TX, RB), NB = (kDirOut + 2 * RB4) / 8;
     float in[2][8];
@@ -217,7 +298,7 @@ __device__ __forceinline__ void dir_ring_conv(DirSums& acc, const DirTaps<RB>& t
     for (int blk = 0; blk < NB; ++blk) {
         if (blk + 1 < NB) fetch(blk + 1);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc.template add<RB>(tp, in[blk & 1][e], 8 * blk + e);
+        for (int e = 0; e < 8; e += 2) acc.template add<RB>(tp, in[blk & 1][e], in[blk & 1][e + 1], 8 * blk + e);
         // Sums formed here, reads one block ahead: left alone, the compiler forms
         // one output after the other (sinking the sums to their stores), with
         // the whole run's inputs live (122 VGPRs at radius 31 instead of 80).
@@ -300,14 +381,12 @@ __device__ __forceinline__ void dir_xy_strip(float* lds, const DirRecord* rec, r
         __syncthreads();
         if (b + 1 < nb) fetch(yb + B);
         {
-            DirSums acc;
+            DirSums<dir_pairs(RB)> acc;
 #pragma unroll
             for (int i = 0; i < (kDirOut + 2 * RB4) / 4; ++i) {
                 const float4 u = raw[xr * W4 + (i & 1) * (W4 / 2) + xt + (i >> 1)];
-                acc.template add<RB>(tx, u.x, 4 * i);
-                acc.template add<RB>(tx, u.y, 4 * i + 1);
-                acc.template add<RB>(tx, u.z, 4 * i + 2);
-                acc.template add<RB>(tx, u.w, 4 * i + 3);
+                acc.template add<RB>(tx, u.x, u.y, 4 * i);
+                acc.template add<RB>(tx, u.z, u.w, 4 * i + 2);
             }
             int row = pos + xr;
             row = row >= RS ? row - RS : row;
@@ -319,7 +398,7 @@ __device__ __forceinline__ void dir_xy_strip(float* lds, const DirRecord* rec, r
         if (b >= M0) {
             int start = pos + 8 * rg - 2 * RB4;
             start = start < 0 ? start + RS : start >= RS ? start - RS : start;
-            DirSums acc;
+            DirSums<dir_pairs(RB)> acc;
             dir_ring_conv<TX, RB>(acc, ty, ring, start, col);
             const int yo = yb - RB4 + 8 * rg;  // wave-uniform, as the rows' bases
             unsigned base = (plane + (unsigned)yo * (unsigned)d.nx) * 4u;
@@ -440,7 +519,7 @@ __device__ __forceinline__ void dir_z_strip(float* ring, const FieldDesc& fd, co
                 for (int v = 0; v < kDirOut; ++v)
                     dl[v] = BufOps<float>::ld_r<kStream>(rdel, live && zo + v < d.nz ? off + (unsigned)v * np * 4u : kBufOOB);
             }
-            DirSums acc;
+            DirSums<dir_pairs(RB)> acc;
             dir_ring_conv<TX, RB>(acc, tz, ring, start, cc);
 #pragma unroll
             for (int v = 0; v < kDirOut; ++v) {
