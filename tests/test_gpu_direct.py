@@ -6,6 +6,10 @@ Tolerance.  The fields and windows are non-negative, so an output is a sum of
 non-negative terms and rounding errors are relative to it element by element:
 per axis at most R + 2 roundings of the running sums, one of the tap and one of
 the stored result, plus two for the decay: |err| <= (3 (R + 4) + 2) 2^-24 v.
+Radius bounds of 8 and more form outputs in pairs, half the products with a
+shared sum: two thirds of the roundings, and terms that exceed the output's own
+only by tap differences, which for these windows (sigma >= 1.25) are below their
+taps near the centre and, further out, small against the fields' background.
 """
 import numpy as np
 import pytest

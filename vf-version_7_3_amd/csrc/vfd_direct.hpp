@@ -319,8 +319,8 @@ template <int A> __device__ __forceinline__ float4 dir_ld4(rsrc_t r, unsigned of
 }
 
 // x and y windows of one strip: TX columns from x0, rows [y0, y1) of plane z.
-// 8 fields 1024x512x128 (R 6 - 19) in 0.99 ms: 4.4 TB/s, and vector instructions
-// for most of that time (0.92 of it one output at a time, 1.08 ms).
+// Bound by vector instructions, 0.96 of its cycles: 8 fields 1024x512x128 (R 6 - 19)
+// in 0.99 ms, 4.4 TB/s (1.08 ms one output at a time).
 template <int TX, int RB>
 __device__ __forceinline__ void dir_xy_strip(float* lds, const DirRecord* rec, rsrc_t rin, rsrc_t rw, const DirDims& d,
                                              int z, int x0, int y0, int y1) {
@@ -419,7 +419,8 @@ __device__ __forceinline__ void dir_xy_strip(float* lds, const DirRecord* rec, r
 }
 
 // The radius bounds compiled: a field takes the smallest that holds its radius.
-// An even step wastes at most one tap a side; beyond 20 (the radius of
+// An even step wastes at most one tap a side (the odd bounds as well: within 2 %
+// either way); beyond 20 (the radius of
 // D = 5 patch^2 a tick is 19) steps of 4.
 #define VFD_DIR_RADII(X) X(2) X(4) X(6) X(8) X(10) X(12) X(14) X(16) X(18) X(20) X(24) X(28) X(31)
 
