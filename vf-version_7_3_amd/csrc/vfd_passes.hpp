@@ -100,11 +100,20 @@ __device__ __forceinline__ bool dir_form(const void* rec) {
 }
 
 // The fields of a launch that the FFT passes do, as a bit mask: those whose
-// record does not have the direct form.  A lane reads a record.
+// record does not have the direct form.  A lane reads a record, in turns where
+// the wave has fewer lanes than the batch has fields: the last wave of a
+// work-group that is no multiple of 64 threads (rows of 576: 216 threads, of
+// 1152: 72, 144 or 216; columns of 72: 144).  Every wave of a work-group must
+// come to the same mask.  Called with the wave's lanes together.
 __device__ __forceinline__ unsigned fft_fields(const FieldBatch& fb, int nfields, unsigned long rec_off) {
-    const int l = (int)(threadIdx.x % 64u);
-    const bool fft = l < nfields && !dir_form((const char*)fb.f[l].work + rec_off);
-    return (unsigned)__ballot(fft);
+    const int l = (int)(threadIdx.x % 64u), lanes = __builtin_popcountll(__ballot(true));
+    unsigned mask = 0;
+    for (int f0 = 0; f0 < nfields; f0 += lanes) {
+        const int f = f0 + l;
+        const bool fft = f < nfields && !dir_form((const char*)fb.f[f].work + rec_off);
+        mask |= (unsigned)__ballot(fft) << f0;
+    }
+    return mask;
 }
 // the n-th set bit of the mask (n < popcount)
 __device__ __forceinline__ unsigned nth_field(unsigned mask, unsigned n) {
