@@ -116,11 +116,13 @@ struct Branches {
     }
 };
 
-// the fields of one batch grouped by shape and form, with the work buffers they own
+// the fields of one batch grouped by shape, with the work buffers they own.  A
+// shape's two forms take turns on its buffers (and so on one stream): admission
+// keeps one buffer per shape for certain, which has to do for both
 struct Group {
     Shape* shape = nullptr;
-    int max_radius = -1;  // direct form: largest radius of the fields; -1: FFT form
-    std::vector<vfd_field> fields;
+    int max_radius = -1;  // largest radius of the direct form's fields
+    std::vector<vfd_field> fft, direct;
 };
 struct Batch {
     std::vector<Group> groups;
@@ -225,26 +227,28 @@ bool trim_pools(vfd_engine* e) {
     return any;
 }
 
-// Group the listed runs' fields by shape and form and reserve their work buffers
+// Group the listed runs' fields by shape and reserve their work buffers
 // (every allocation happens here, never while a stream is being captured).
 int build_batch(vfd_engine* e, const std::vector<int>& run_ids, Batch* bt) {
-    std::map<std::pair<ShapeKey, bool>, Group> groups;
+    std::map<ShapeKey, Group> groups;
     for (int id : run_ids) {
         auto it = e->runs.find(id);
         if (it == e->runs.end()) return set_error(VFD_ERR_NOTFOUND, "step: unknown run %d", id);
         Run& r = it->second;
         for (int f = 0; f < r.nfields; ++f) {
-            Group& g = groups[{r.key, r.radius[f] >= 0}];
+            Group& g = groups[r.key];
             g.max_radius = std::max(g.max_radius, r.radius[f]);
-            g.fields.push_back(vfd_field{r.field[f], r.field[f], nullptr, r.kspec[f], 0.0, 0, 0});
+            (r.radius[f] >= 0 ? g.direct : g.fft)
+                .push_back(vfd_field{r.field[f], r.field[f], nullptr, r.kspec[f], 0.0, 0, 0});
         }
     }
     for (auto& kv : groups) {
-        const ShapeKey& key = kv.first.first;
+        const ShapeKey& key = kv.first;
         Shape& s = e->shapes[key];
         Held h;
         const int by_bytes = (int)std::max<size_t>(1, group_work_bytes() / s.plan.work_bytes);
-        const int want = std::min({(int)kv.second.fields.size(), kMaxFieldsPerLaunch, by_bytes});
+        const int nf = (int)(kv.second.fft.size() + kv.second.direct.size());
+        const int want = std::min({nf, kMaxFieldsPerLaunch, by_bytes});
         if (acquire(e, s, want, &h) < 1) {
             release(h);
             for (auto& hh : bt->held) release(hh);
@@ -268,7 +272,8 @@ void release_batch(Batch* bt) {
 
 // Launch `ticks` ticks of a built batch: shapes run on branch streams forked
 // from / joined to `st` with events (also valid while `st` is captured);
-// within a shape, fields go in chunks of the reserved work-buffer count.
+// within a shape, fields go in chunks of the reserved work-buffer count, those
+// of the FFT form first, then those of the direct form.
 int launch_batch(Batch& bt, int ticks, hipStream_t st, Branches& br) {
     const int ng = (int)bt.groups.size();
     if (ng == 0) return VFD_OK;
@@ -279,29 +284,31 @@ int launch_batch(Batch& bt, int ticks, hipStream_t st, Branches& br) {
     for (int gi = 0; gi < ng; ++gi) {
         Group& g = bt.groups[gi];
         Shape& s = *g.shape;
-        std::vector<vfd_field>& fl = g.fields;
         const Held& h = bt.held[gi];
+        const size_t nbuf = h.idx.size();
         // the direct form keeps one real field between its passes: a work buffer
         // (the FFT form's padded half spectrum) has room for several
-        const bool direct = g.max_radius >= 0;
         const size_t slot = (s.plan.field_bytes + 255) / 256 * 256;
-        const size_t per_buf = direct ? std::max<size_t>(1, s.plan.work_bytes / slot) : 1;
-        size_t k = h.idx.size() * per_buf;
-        if (direct) k = std::min<size_t>({k, (size_t)kMaxFieldsPerLaunch, std::max<size_t>(1, group_work_bytes() / slot)});
+        const size_t kdir = std::min<size_t>({nbuf * std::max<size_t>(1, s.plan.work_bytes / slot),
+                                              (size_t)kMaxFieldsPerLaunch,
+                                              std::max<size_t>(1, group_work_bytes() / slot)});
         hipStream_t gs = fork ? br.aux[gi % kAuxStreams] : st;
         if (fork) {
             if (int rc = hip_check(hipStreamWaitEvent(gs, br.fork, 0), "fork wait")) return rc;
         }
-        for (int t = 0; t < ticks; ++t)
-            for (size_t c = 0; c < fl.size(); c += k) {
-                const int n = (int)std::min(k, fl.size() - c);
-                // spread over the buffers first, then over the slots of each
-                for (int i = 0; i < n; ++i)
-                    fl[c + i].work = (char*)s.pool[h.idx[i % h.idx.size()]] + i / h.idx.size() * slot;
-                const int rc = direct ? plan_diffuse_direct(s.plan, fl.data() + c, n, g.max_radius, 0, 5, gs)
-                                      : plan_diffuse(s.plan, fl.data() + c, n, gs, Form::fft);
-                if (rc) return rc;
+        for (int t = 0; t < ticks; ++t) {
+            for (size_t c = 0; c < g.fft.size(); c += nbuf) {
+                const int n = (int)std::min(nbuf, g.fft.size() - c);
+                for (int i = 0; i < n; ++i) g.fft[c + i].work = s.pool[h.idx[i]];
+                if (int rc = plan_diffuse(s.plan, g.fft.data() + c, n, gs, Form::fft)) return rc;
             }
+            for (size_t c = 0; c < g.direct.size(); c += kdir) {
+                const int n = (int)std::min(kdir, g.direct.size() - c);
+                // spread over the buffers first, then over the slots of each
+                for (int i = 0; i < n; ++i) g.direct[c + i].work = (char*)s.pool[h.idx[i % nbuf]] + i / nbuf * slot;
+                if (int rc = plan_diffuse_direct(s.plan, g.direct.data() + c, n, g.max_radius, 0, 5, gs)) return rc;
+            }
+        }
         if (fork) {
             if (int rc = hip_check(hipEventRecord(br.join[gi % kAuxStreams], gs), "join")) return rc;
             if (int rc = hip_check(hipStreamWaitEvent(st, br.join[gi % kAuxStreams], 0), "join wait")) return rc;
