@@ -97,3 +97,34 @@ def test_two_shapes_with_both_forms_in_one_batch(vfd, orc):
         for x, y in ((a1, a2), (b1, b2)):
             for f, (p, q) in enumerate(zip(_fields(eng, x, len(RADII)), _fields(eng, y, len(RADII)))):
                 assert np.array_equal(p, q), f
+
+
+def test_run_is_whole_when_its_id_is_returned(vfd, orc):
+    """A run is written and ticked at once on a stream that does not wait for the
+    null stream: its fields and the last field's record have to be there already
+    (an admission leaves no work queued)."""
+    import torch
+    import vfd.engine as em
+    shape, radii = (64, 128, 128), (31, 5, 36, 12, 8)   # ends in a field of the direct form
+    print("case run used at once on a side stream", flush=True)
+    s2, dec = [_s2(r) for r in radii], [DECAY] * len(radii)
+    us = [torch.from_numpy(orc.synth_field(shape, 71 + f, nsrc=5)).cuda() for f in range(len(radii))]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    got = []
+    with em.Engine(4 << 30) as eng:
+        for rep in range(4):
+            rid = eng.create_run(shape, s2, dec)
+            assert torch.cuda.default_stream().query()
+            for f in reversed(range(len(radii))):
+                eng.write_field(rid, f, us[f], stream=side)
+            eng.step([rid], stream=side)
+            side.synchronize()
+            out = [eng.read_field(rid, f, stream=side) for f in range(len(radii))]
+            side.synchronize()
+            got.append([o.cpu().numpy() for o in out])
+    for f, r in enumerate(radii):
+        ref = orc.direct_separable(us[f].cpu().numpy(), s2[f], DECAY)
+        assert orc.rel_l2(got[0][f], ref) <= 1e-5, r
+        for g in got[1:]:
+            assert np.array_equal(g[f], got[0][f]), r

@@ -554,8 +554,12 @@ static int run_create(vfd_engine* e, const vfd_run_desc* d, int* run_id, double 
             if (!rc && r.radius[f] >= 0)
                 rc = hip_check(hipMemcpyAsync(kp, fp, kDirRecordBytes, hipMemcpyDeviceToDevice, nullptr), "run record");
         }
-        if (!rc) rc = hip_check(hipMemset(fp, 0, plan.field_bytes), "run field clear");
+        if (!rc) rc = hip_check(hipMemsetAsync(fp, 0, plan.field_bytes, nullptr), "run field clear");
     }
+    // the records and the clears are done before anyone can name the run: the
+    // streams it is written and ticked on (the server's, the branches', callers'
+    // own) need not wait for the null stream
+    if (!rc) rc = hip_check(hipStreamSynchronize(nullptr), "run create sync");
     std::vector<void*> frees;
     size_t unreserve = 0;
     {
