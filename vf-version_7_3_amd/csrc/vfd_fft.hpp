@@ -117,12 +117,8 @@ constexpr Rot best_rot(double c, double s, double target = 1.0) {
         }
     return best;
 }
-// W16^1 and the radix-3 pair (-1/2, sqrt(3)/2), both directions
+// W16^1, both directions (W8 and the radix-3 sine go as hi + lo, below)
 constexpr Rot kW16 = best_rot(0.92387953251128675613, 0.38268343236508977173);
-constexpr Rot kW3 = best_rot(-0.5, 0.86602540378443864676);
-// W8^1 = (1 - i)/sqrt(2): the plain rounding (near 45 degrees the FP32 lattice
-// moves |w|^2 in steps of about 8e-8)
-constexpr Rot kW8 = Rot{(float)0.70710678118654752440, (float)0.70710678118654752440};
 }  // namespace ce
 
 // ------------------------------------------------------------ butterflies
@@ -154,48 +150,46 @@ template <bool INV, typename T> struct Bfly<4, INV, T> {
 // round trip gave each FP32 inverse pass a gain of its own, and the drift from
 // FP64 over many ticks grew: 100-tick rel-L2 9.8e-6 against 6.9e-6.)
 template <typename T, bool INV> struct Rots {
-    static constexpr T w8c = T(0.70710678118654752440), w8s = T(0.70710678118654752440);
     static constexpr T w16c = T(0.92387953251128675613), w16s = T(0.38268343236508977173);
-    static constexpr T w3c = T(-0.5), w3s = T(0.86602540378443864676);
 };
 template <bool INV> struct Rots<float, INV> {
-    static constexpr ce::Rot w8 = ce::kW8, w16 = ce::kW16, w3 = ce::kW3;
-    static constexpr float w8c = w8.c, w8s = w8.s, w16c = w16.c, w16s = w16.s, w3c = w3.c, w3s = w3.s;
+    static constexpr ce::Rot w16 = ce::kW16;
+    static constexpr float w16c = w16.c, w16s = w16.s;
 };
 
-// FP32: 1/sqrt(2) as hi + lo.  The FP32 value alone is the only pair near 45
-// degrees and has |w|^2 - 1 = -3.4e-8, the same on every path through a W8
-// rotation; (x -+ y) hi + (x -+ y) lo carries no such gain.
-constexpr float kRsqrt2Hi = 0.70710678118654752440f;
-constexpr float kRsqrt2Lo = (float)(0.70710678118654752440 - (double)kRsqrt2Hi);
-__device__ __forceinline__ float rsqrt2_mul(float p) { return fmaf(p, kRsqrt2Hi, p * kRsqrt2Lo); }
-// the same for sin(2 pi/3) of the radix-3 butterfly (its best FP32 pair is
-// off by -1.1e-8 in |w|^2).  W16's pair is left single (+7e-9): carrying it
-// as hi + lo too made the step 0.5 % slower for a smaller rel-L2 (100-tick
-// precision run 3.4e-6 -> 2.6e-6) and a larger mass drift (2.0e-6 -> 2.5e-6).
-constexpr double kS3 = 0.86602540378443864676;
-constexpr float kS3Hi = (float)kS3, kS3Lo = (float)(kS3 - (double)(float)kS3);
+// 1/sqrt(2) and sin(2 pi/3) as hi + lo.  FP32: the single value is the only pair
+// near 45 degrees and has |w|^2 - 1 = -3.4e-8, the same on every path through a
+// W8 rotation; (x -+ y) hi + (x -+ y) lo carries no such gain, and the radix-3
+// sine's best FP32 pair is off by -1.1e-8.  W16's pair is left single (+7e-9):
+// carrying it as hi + lo too made the step 0.5 % slower for a smaller rel-L2
+// (100-tick precision run 3.4e-6 -> 2.6e-6) and a larger mass drift (2.0e-6 ->
+// 2.5e-6).  FP64: the single values are off by -6.8e-17 and +5.8e-17 of
+// themselves, and radix-8 plans cross more W8 rotations than the radix-16 ones;
+// as hi + lo their error is no larger than radix 16 had with single values.
+template <typename T> struct HiLo;
+template <> struct HiLo<float> {
+    static constexpr double kR2 = 0.70710678118654752440, kS3 = 0.86602540378443864676;
+    static constexpr float r2 = (float)kR2, r2_lo = (float)(kR2 - (double)r2);
+    static constexpr float s3 = (float)kS3, s3_lo = (float)(kS3 - (double)s3);
+};
+template <> struct HiLo<double> {
+    static constexpr double r2 = 0.70710678118654752440, r2_lo = -4.833646656726457e-17;
+    static constexpr double s3 = 0.86602540378443864676, s3_lo = 5.0175421109034514e-17;
+};
+__device__ __forceinline__ float fma_(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return fma(a, b, c); }
+template <typename T> __device__ __forceinline__ T rsqrt2_mul(T p) { return fma_(p, HiLo<T>::r2, p * HiLo<T>::r2_lo); }
+template <typename T> __device__ __forceinline__ T s3_mul(T p) { return fma_(p, HiLo<T>::s3, p * HiLo<T>::s3_lo); }
 
-// multiply by W8^1 = (1 - i)/sqrt(2) (fwd) / (1 + i)/sqrt(2) (inv), as the
-// pair (a, b) ~ (1/sqrt(2), 1/sqrt(2)): c (a -+ i b)
+// multiply by W8^1 = (1 - i)/sqrt(2) (fwd) / (1 + i)/sqrt(2) (inv)
 template <bool INV, typename T> __device__ __forceinline__ cx<T> w8_1(cx<T> c) {
-    if constexpr (sizeof(T) == 4) {
-        return INV ? cx<T>{rsqrt2_mul(c.x - c.y), rsqrt2_mul(c.y + c.x)}
-                   : cx<T>{rsqrt2_mul(c.x + c.y), rsqrt2_mul(c.y - c.x)};
-    } else {
-        constexpr T a = Rots<T, INV>::w8c, b = Rots<T, INV>::w8s;
-        return INV ? cx<T>{c.x * a - c.y * b, c.y * a + c.x * b} : cx<T>{c.x * a + c.y * b, c.y * a - c.x * b};
-    }
+    return INV ? cx<T>{rsqrt2_mul(c.x - c.y), rsqrt2_mul(c.y + c.x)}
+               : cx<T>{rsqrt2_mul(c.x + c.y), rsqrt2_mul(c.y - c.x)};
 }
-// multiply by W8^3 = (-1 - i)/sqrt(2) (fwd) / (-1 + i)/sqrt(2) (inv): c (-a -+ i b)
+// multiply by W8^3 = (-1 - i)/sqrt(2) (fwd) / (-1 + i)/sqrt(2) (inv)
 template <bool INV, typename T> __device__ __forceinline__ cx<T> w8_3(cx<T> c) {
-    if constexpr (sizeof(T) == 4) {
-        return INV ? cx<T>{rsqrt2_mul(-c.x - c.y), rsqrt2_mul(c.x - c.y)}
-                   : cx<T>{rsqrt2_mul(c.y - c.x), rsqrt2_mul(-c.y - c.x)};
-    } else {
-        constexpr T a = Rots<T, INV>::w8c, b = Rots<T, INV>::w8s;
-        return INV ? cx<T>{-c.x * a - c.y * b, c.x * b - c.y * a} : cx<T>{c.y * b - c.x * a, -c.y * a - c.x * b};
-    }
+    return INV ? cx<T>{rsqrt2_mul(-c.x - c.y), rsqrt2_mul(c.x - c.y)}
+               : cx<T>{rsqrt2_mul(c.y - c.x), rsqrt2_mul(-c.y - c.x)};
 }
 
 template <bool INV, typename T> struct Bfly<8, INV, T> {
@@ -258,20 +252,12 @@ template <bool INV, typename T> struct Bfly<16, INV, T> {
 
 template <bool INV, typename T> struct Bfly<3, INV, T> {
     static __device__ __forceinline__ void run(cx<T>* v) {
-        constexpr T c3 = Rots<T, INV>::w3c;  // cos(2 pi/3) = -1/2
-        constexpr T s3 = Rots<T, INV>::w3s;  // sin(2 pi/3)
         cx<T> s = cadd(v[1], v[2]), d = csub(v[1], v[2]);
         cx<T> a0 = v[0];
         v[0] = cadd(a0, s);
-        cx<T> t, sd;
-        if constexpr (sizeof(T) == 4) {
-            // FP32: c3 = -1/2 exactly, s3 as hi + lo
-            t = cx<T>{fmaf(-0.5f, s.x, a0.x), fmaf(-0.5f, s.y, a0.y)};
-            sd = cx<T>{fmaf(d.x, kS3Hi, d.x * kS3Lo), fmaf(d.y, kS3Hi, d.y * kS3Lo)};
-        } else {
-            t = cx<T>{a0.x + c3 * s.x, a0.y + c3 * s.y};
-            sd = cscale(d, s3);
-        }
+        // cos(2 pi/3) = -1/2
+        const cx<T> t{fma_(T(-0.5), s.x, a0.x), fma_(T(-0.5), s.y, a0.y)};
+        const cx<T> sd{s3_mul(d.x), s3_mul(d.y)};
         // fwd: y1 = t - i s3 d ; y2 = t + i s3 d
         cx<T> m = mul_mi<INV>(sd);
         v[1] = cadd(t, m);

@@ -24,7 +24,9 @@ namespace vfd {
 //  FP64 (a complex value takes 4 registers): z pass of 4 fields 256x128x64
 //   252 -> 157 us, y inverse 97 -> 76, x passes 51 + 60 -> 49 + 49; a tick of 8
 //   fields 130x100x40 394 -> 313 us, of 2 fields 512x256x128 1982 -> 1550 us;
-//   one stage more per transform: rel-L2 of a tick 9.3e-16 for 8.7e-16;
+//   one stage more per transform, no less accurate with the butterflies'
+//   constants as hi + lo (HiLo; a round trip's rel-L2 over 14 boxes 0.95 of
+//   radix 16 with single values, 1.04 without hi + lo);
 //  FP32 (rows with 512-thread, columns with 256-thread work-groups): ticks of
 //   301x187x75 (8 fields) 1418 -> 1165 us, 560x51x90 (6) 711 -> 497, 140x100x40
 //   (8) 187 -> 160, 1100x600x36 (2) 1992 -> 1713.
