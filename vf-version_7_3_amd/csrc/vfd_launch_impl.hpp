@@ -28,14 +28,22 @@ namespace vfd {
 //   constants as hi + lo (HiLo; a round trip's rel-L2 over 14 boxes 0.95 of
 //   radix 16 with single values, 1.04 without hi + lo);
 //  FP32 (rows with 512-thread, columns with 256-thread work-groups): ticks of
-//   301x187x75 (8 fields) 1418 -> 1165 us, 560x51x90 (6) 711 -> 497, 140x100x40
+//   301x187x75 (8 fields) 1418 -> 1314 us, 560x51x90 (6) 711 -> 497, 140x100x40
 //   (8) 187 -> 160, 1100x600x36 (2) 1992 -> 1713.
 // Columns of 144 keep radix 16 (16 9 in three stages against 8 2 3 3 in four,
 // with only 16 columns a work-group): fused z pass 660 against 802 us.
+// FP32 lengths of 16, 48 and 80 keep radix 16, in 256 threads: radix 8 does their
+// 16 as 8 2, whose rotations by W16 come from the table in single FP32 values and
+// are a gain (rel-L2 of a streamed-spectrum tick of 16^3, 48^3 1.10e-7, 0.98e-7
+// against 1.31e-7, 1.08e-7; 301x187x75 1.14 against 1.15).  8 fields of 16^3, 48^3,
+// 80^3: 23.6, 54.5, 160 us; radix 16 in 512 threads 27, 59, 214; radix 8 23, 47, 133.
+template <typename T, int Q> constexpr bool one_r16() { return sizeof(T) == 4 && (Q == 16 || Q == 48 || Q == 80); }
 #ifdef VFD_ROW_TU
-template <typename T, int Q> constexpr int single_var() { return 1; }
+template <typename T, int Q> constexpr int single_var() { return one_r16<T, Q>() ? 3 : 1; }
 #else
-template <typename T, int Q> constexpr int single_var() { return sizeof(T) == 4 && Q == 144 ? 0 : 2; }
+template <typename T, int Q> constexpr int single_var() {
+    return one_r16<T, Q>() ? 3 : sizeof(T) == 4 && Q == 144 ? 0 : 2;
+}
 #endif
 
 // resident work-groups per CU for a kernel (callers cache it per instantiation)
