@@ -62,7 +62,9 @@ enum { VFD_PAD_CONSTANT_VF = 3, VFD_PAD_ZERO = 100 };
  *                        the same operator to FP32 rounding.  The form is found
  *                        on the device from the tables of the call, on every
  *                        call, so a table copied, moved or edited by any means
- *                        runs the form its own contents select.
+ *                        runs the form its own contents select; except that
+                        a plan whose own vfd_gauss_spectrum calls were all beyond
+                        radius 31 runs the FFT passes on every table.
  *                        VFD_PAD_ZERO plans only. */
 enum { VFD_KSPEC_REAL = 0, VFD_KSPEC_COMPLEX_STD = 1, VFD_KSPEC_SEPARABLE = 2 };
 

@@ -34,7 +34,8 @@ struct Plan {
     size_t rec_off;
     // which tables the plan's own vfd_gauss_spectrum has made: bit 0 within the
     // direct form's radius, bit 1 beyond.  A hint for the launch shape of the FFT
-    // passes (Records), never for what they do; accessed atomically
+    // passes (Records); bit 1 alone: whole ticks are the FFT form's, which does any
+    // table.  Accessed atomically
     mutable int tables;
 };
 

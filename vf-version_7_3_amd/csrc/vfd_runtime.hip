@@ -465,6 +465,14 @@ int plan_diffuse_passes(const Plan& p, const vfd_field* fields, int nfields, int
     if (int rc = check_fields(fields, nfields)) return rc;
     if (lo < 0 || hi > 5 || lo >= hi) return set_error(VFD_ERR_INVALID, "diffuse: bad pass range [%d,%d)", lo, hi);
     if (nfields == 0) return VFD_OK;
+    // A plan that has made wide tables only runs whole ticks in the FFT form, which
+    // does any table: classify, the two direct launches and the passes' record tests
+    // would find nothing, 16 % of a tick of 8 fields 64x64x32 of radius 32 (53.4
+    // against 62.0 us; one field 33.5 and 39.1; 8 fields 128x128x64 of radius 36 204
+    // and 217).  Single passes (vfd_diffuse_pass) keep to the records: a plan's tables
+    // may change between two of them.
+    if (form == Form::by_table && lo == 0 && hi == 5 && __atomic_load_n(&p.tables, __ATOMIC_RELAXED) == 2)
+        form = Form::fft;
     return p.prec == VFD_F32 ? run_tick<float>(p, fields, nfields, lo, hi, st, epi, -1, form)
                              : run_tick<double>(p, fields, nfields, lo, hi, st, epi);
 }
