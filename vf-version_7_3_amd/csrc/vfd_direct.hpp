@@ -121,7 +121,12 @@ dir_classify_kernel(const FieldBatch fb, DirDims d) {
     if (bad) bad_s = 1;
     __syncthreads();
     if (tid < kWave) {  // one wave: lanes 0 .. 31 hold a tap each
-        const double v = tid < kDirTaps ? h[tid] : 0.0;
+        // the taps go to FP32 with their sum near 1 (within 0.75 .. 1.5, where a
+        // normalized window's is already), the power of two back into the gain: a
+        // table may hold any part of the kernel's magnitude in any of its factors
+        int e2 = 0;
+        if (gmax > 0.0 && frexp(gmax, &e2) < 0.75) --e2;
+        const double v = tid < kDirTaps ? ldexp(h[tid], -e2) : 0.0;
         double hmax = fabs(v);
         for (int m = kDirTaps / 2; m > 0; m >>= 1) hmax = fmax(hmax, __shfl_xor(hmax, m));
         const unsigned long long big = __ballot(fabs(v) > 1e-13 * hmax) & 0xffffffffull;
@@ -138,7 +143,7 @@ dir_classify_kernel(const FieldBatch fb, DirDims d) {
         }
         if (tid < kDirTaps) rec->ax[ax].tap[tid] = in ? (float)v : 0.0f;
         if (tid == 0) {
-            rec->ax[ax].gain = pos && sr > 0.0 ? se / sr : 1.0;
+            rec->ax[ax].gain = ldexp(pos && sr > 0.0 ? se / sr : 1.0, e2);
             rec->ax[ax].radius = !bad_s && R <= P - n ? R : -1;
             if (ax == 0) rec->scale = tab[0] * (double)d.px * (double)d.py * (double)d.pz;
         }
@@ -466,7 +471,7 @@ __device__ __forceinline__ void dir_z_strip(float* ring, const FieldDesc& fd, co
     const rsrc_t rw = make_rsrc(fd.work, d.bytes), rout = make_rsrc(fd.out, d.bytes);
     DirTaps<RB> tz;
     tz.load(&rec->ax[2]);
-    // the decay (and the taps' FP32 rounding, see classify) as hi + lo
+    // the decay (and the taps' power of two and FP32 rounding, see classify) as hi + lo
     const double fac = rec->scale * rec->ax[0].gain * rec->ax[1].gain * rec->ax[2].gain;
     const float fh = (float)fac, fl = (float)(fac - (double)fh);
     const unsigned np = (unsigned)d.ny * (unsigned)d.nx;

@@ -106,7 +106,9 @@ struct XlDesc {
 constexpr int kDirMaxR = 31;
 constexpr int kDirHalfMax = 2304;  // half the longest box axis (dir_classify's LDS): the longest compiled length
 struct DirAxis {
-    double gain;               // exact window sum / sum of the FP32 taps (1 where not all taps are >= 0)
+    // exact window sum / sum of the FP32 taps (not all taps >= 0: 1), times the power
+    // of two that the taps were divided by
+    double gain;
     int radius;                // -1: the axis' table is not a short window
     float tap[kDirMaxR + 1];   // h_0 .. h_R, then zeros
 };
