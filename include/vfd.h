@@ -63,8 +63,10 @@ enum { VFD_PAD_CONSTANT_VF = 3, VFD_PAD_ZERO = 100 };
  *                        on the device from the tables of the call, on every
  *                        call, so a table copied, moved or edited by any means
  *                        runs the form its own contents select; except that
-                        a plan whose own vfd_gauss_spectrum calls were all beyond
-                        radius 31 runs the FFT passes on every table.
+ *                        a plan whose own vfd_gauss_spectrum calls were all beyond
+ *                        radius 31 runs the FFT passes on every table.  A plan
+ *                        that has made short tables only expects no others: wide
+ *                        ones of another plan run correctly, up to 17 % slower.
  *                        VFD_PAD_ZERO plans only. */
 enum { VFD_KSPEC_REAL = 0, VFD_KSPEC_COMPLEX_STD = 1, VFD_KSPEC_SEPARABLE = 2 };
 
@@ -131,8 +133,12 @@ int vfd_diffuse(const vfd_plan* plan, const vfd_field* fields, int nfields, void
  * for per-pass timing.  In the XLAST order the same five indices run z R2C,
  * y forward, the fused x pass, y inverse and z C2R.  A separable FP32 field of
  * the direct form is done by the first pass (x and y windows, into work) and the
- * last (z window); the passes between leave it alone.  vfd_plan_pass_bytes gives the algorithmic HBM bytes
- * of one pass for one field (sum over passes = bytes_per_field_tick). */
+ * last (z window); the passes between leave it alone.  Which
+ * form that is is found by VFD_PASS_XFWD and kept in work: the other passes, and
+ * the parts below, follow it on the same fields and work arrays, in one plan.
+ * vfd_plan_pass_bytes gives the algorithmic HBM bytes of one pass of the FFT form
+ * for one field (sum over passes = bytes_per_field_tick); a field of the direct
+ * form moves 16 bytes a voxel instead, 8 in its first pass and 8 in its last. */
 enum { VFD_PASS_XFWD = 0, VFD_PASS_YFWD = 1, VFD_PASS_ZCONV = 2, VFD_PASS_YINV = 3, VFD_PASS_XINV = 4 };
 /* Parts of the z pass, for per-kernel timing: the direct z pass for radius
  * bound 8, 12 and 16 (FP32 separable plans; no launch otherwise; VFD_PASS_ZCONV
