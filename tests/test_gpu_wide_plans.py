@@ -41,3 +41,32 @@ def test_wide_plans_skip_the_direct_form(vfd, orc):
     got = _tick(plan, ud, wide, work)
     assert not bool((work[-RECORD:] == 0xA5).all())
     assert float(np.linalg.norm(got - orc.direct_separable(u, _s2(36), 0.97)) / np.linalg.norm(got)) <= 1e-5
+
+
+@pytest.mark.parametrize("radii", [(36,) * 8, (36, 6) * 4], ids=["wide", "both"])
+def test_fused_epilogues_of_wide_windows(vfd, radii):
+    """The chem update and the downsample in the last pass against the separate
+    calls on the same inputs: the same bits, for plans of wide tables (FFT passes
+    without records) and of both kinds (with)."""
+    import torch
+    print(f"case epilogues {radii}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    plan = vfd.Plan(SHAPE, kspec_format=vfd.KSPEC_SEPARABLE)
+    rand = lambda: torch.rand(SHAPE, generator=g, device="cuda")
+    u, d, col, ela, decay = [rand() for _ in radii], [rand() for _ in radii], rand(), rand(), [0.3] * 8
+    ks = [plan.gauss_spectrum(_s2(r), 0.97) for r in radii]
+    entries = lambda out: [{"in": a, "out": o, "work": plan.new_work(), "kspec": k} for a, o, k in zip(u, out, ks)]
+    new = lambda: [torch.empty_like(x) for x in u]
+    t, levels, fused = new(), new(), new()
+    grads, fused_grads = [torch.empty_like(col) for _ in range(3)], [torch.empty_like(col) for _ in range(3)]
+    plan.diffuse(entries(t))
+    vfd.chem_update(t, [x.clone() for x in d], levels, decay, col, ela, grads)
+    plan.diffuse_update(entries(fused), d, decay, col, ela, fused_grads)
+    out, want = new(), [vfd.sample_chem(x, c, 3) for c, x in enumerate(t)]
+    vis = [torch.full_like(w, -1.0) for w in want]
+    plan.diffuse_sample(entries(out), list(range(8)), 3, vis)
+    torch.cuda.synchronize()
+    for i in range(8):
+        assert torch.equal(fused[i], levels[i]) and not d[i].any(), i
+        assert torch.equal(out[i], t[i]) and torch.equal(vis[i], want[i]), i
+    assert all(torch.equal(a, b) for a, b in zip(fused_grads, grads))
