@@ -55,3 +55,38 @@ def test_single_tick_gain_of_one_radix_16_lengths(vfd, orc):
         gains.append(float(((out.cpu().numpy() - ref) * ref).sum() / (ref * ref).sum()))
     print(f"  gain {np.mean(gains):.2e}", flush=True)
     assert abs(np.mean(gains)) <= 5.2e-8
+
+
+def test_double_tick_has_no_gain(vfd):
+    """FP64 ticks against long double.  A window that is normalized to 1 in more than
+    FP64 has a DFT of exactly 1 at zero frequency, where most of the field is; in FP64
+    its sum and quotients miss 1 by up to some 5e-16 over three axes, by another
+    amount for every sigma.  Left are the product of the tables and the decay, a few
+    roundings of either sign at each frequency: bound, two roundings, 2.2e-16."""
+    import torch
+    shape, L = (64, 64, 64), np.longdouble
+    print("case double tick gain", flush=True)
+    plan = vfd.Plan(shape, precision=vfd.F64, kspec_format=vfd.KSPEC_SEPARABLE)
+    rng = np.random.default_rng(8)
+    worst = 0.0
+    for s2 in (1.1, 1.7, 2.9, 3.7, 5.3, 7.1, 8.3, 9.7):
+        u = rng.lognormal(-2.0, 1.0, shape)
+        radius = int(np.ceil(6.0 * np.sqrt(s2)))
+        j = np.arange(-radius, radius + 1).astype(L)
+        g = np.exp(-j * j / (2 * L(s2)))
+        g /= g.sum()
+        ref = u.astype(L)
+        for ax in range(3):
+            n = shape[ax]
+            m = np.zeros((n, n), dtype=L)
+            for d in range(-radius, radius + 1):
+                m += np.diag(np.full(n - abs(d), g[d + radius], dtype=L), d)
+            ref = np.moveaxis(np.tensordot(m, np.moveaxis(ref, ax, 0), 1), 0, ax)
+        out = torch.empty(shape, dtype=torch.float64, device="cuda")
+        plan.diffuse([{"in": torch.from_numpy(u).cuda(), "out": out, "work": plan.new_work(),
+                       "kspec": plan.gauss_spectrum(s2, 1.0)}])
+        torch.cuda.synchronize()
+        gain = float(((out.cpu().numpy().astype(L) - ref) * ref).sum() / (ref * ref).sum())
+        print(f"  sigma^2 {s2}: gain {gain:.2e}", flush=True)
+        worst = max(worst, abs(gain))
+    assert worst <= 2.0 ** -52

@@ -715,17 +715,19 @@ __global__ void gauss_product_kernel(T* __restrict__ out, const double* __restri
     out[i] = kx < hx ? (T)(((gx[kx] * gy[ky]) * scale) * gz[kz]) : T(0);
 }
 
-// the normalized window g_j, |j| <= R = ceil(6 sigma), as g[j + R]
-static void gauss_window(double sigma2, std::vector<double>& g) {
+// the normalized window g_j, |j| <= R = ceil(6 sigma), as g[j + R].  In long
+// double as its DFT: the roundings of an FP64 sum and quotient are a gain of the
+// whole field (5e-16 over three axes, most of an FP64 tick's error)
+static void gauss_window(double sigma2, std::vector<long double>& g) {
     const int R = (int)std::ceil(6.0 * std::sqrt(sigma2));
-    g.assign(2 * R + 1, 0.0);
-    double s = 0.0;
-    for (int j = -R; j <= R; ++j) s += (g[j + R] = std::exp(-(double)j * j / (2.0 * sigma2)));
+    g.assign(2 * R + 1, 0.0L);
+    long double s = 0.0L;
+    for (int j = -R; j <= R; ++j) s += (g[j + R] = expl(-(long double)j * j / (2.0L * (long double)sigma2)));
     for (auto& v : g) v /= s;
 }
 
 static void gauss_dft(double sigma2, int p, int nk, std::vector<double>& out) {
-    std::vector<double> g;
+    std::vector<long double> g;
     gauss_window(sigma2, g);
     const int R = ((int)g.size() - 1) / 2;
     out.assign(nk, 0.0);
@@ -734,7 +736,7 @@ static void gauss_dft(double sigma2, int p, int nk, std::vector<double>& out) {
         long double acc = 0.0L;
         for (int j = -R; j <= R; ++j) {
             long e = (((long)j * k) % p + p) % p;
-            acc += (long double)g[j + R] * cosl(tp * (long double)e / (long double)p);
+            acc += g[j + R] * cosl(tp * (long double)e / (long double)p);
         }
         out[k] = (double)acc;
     }
@@ -763,11 +765,11 @@ int plan_gauss_spectrum(const Plan& p, double sigma2, double decay, void* d_kspe
         std::copy(gy.begin(), gy.end(), tab.begin() + 1 + p.hx);
         std::copy(gz.begin(), gz.end(), tab.begin() + 1 + p.hx + p.py);
         // the z window for the direct z pass: R, then g_0 .. g_min(R, kZDirectMaxR)
-        std::vector<double> win;
+        std::vector<long double> win;
         gauss_window(sigma2, win);
         const size_t g0 = 1 + p.hx + p.py + p.pz;
         tab[g0] = (double)R;
-        for (int j = 0; j <= std::min(R, kZDirectMaxR); ++j) tab[g0 + 1 + j] = win[R + j];
+        for (int j = 0; j <= std::min(R, kZDirectMaxR); ++j) tab[g0 + 1 + j] = (double)win[R + j];
         if (R <= kZDirectMaxR) {
             // the direct pass multiplies by the taps rounded to FP32; g_0 takes
             // up their rounding so that g_0 + 2 sum_j g_j stays 1 to FP32
