@@ -90,3 +90,38 @@ def test_double_tick_has_no_gain(vfd):
         print(f"  sigma^2 {s2}: gain {gain:.2e}", flush=True)
         worst = max(worst, abs(gain))
     assert worst <= 2.0 ** -52
+
+
+@pytest.mark.parametrize("q", [16, 48, 80])
+def test_one_radix_16_lengths_on_every_axis(vfd, orc, q):
+    """FP32 rows of q, columns of q whole and split from 2 q, fused and not, in
+    batches whose last tile is partial (q + 1 columns), with the streamed spectrum,
+    wide separable tables (q of room for a radius of 36) and as plain transforms.
+    Tolerance: rel-L2 1e-5 against the FP64 oracle, the transforms' eps log2 N."""
+    import torch
+    print(f"case lengths of {q}", flush=True)
+    cases = [((q - 8, q, q), (q, 2 * q, 2 * q), vfd.KSPEC_REAL, 1.2), ((q, q - 8, q), (2 * q, q, 2 * q), vfd.KSPEC_REAL, 1.2)]
+    if q > 36:
+        cases.append(((q, q, q), (2 * q,) * 3, vfd.KSPEC_SEPARABLE, (35.5 / 6.0) ** 2))
+    for shape, box, fmt, s2 in cases:
+        plan = vfd.Plan(shape, box, vfd.F32, kspec_format=fmt)
+        us = [orc.synth_field(shape, 40 + f, nsrc=5) for f in range(3)]
+        outs = [torch.empty(shape, device="cuda") for _ in us]
+        table = plan.gauss_spectrum(s2, 0.97)
+        plan.diffuse([{"in": torch.from_numpy(u).cuda(), "out": o, "work": plan.new_work(), "kspec": table}
+                      for u, o in zip(us, outs)])
+        torch.cuda.synchronize()
+        for u, o in zip(us, outs):
+            assert orc.rel_l2(o.cpu().numpy(), orc.direct_separable(u, s2, 0.97)) <= 1e-5, (shape, box)
+    box = (q, q, 2 * q)
+    plan = vfd.Plan(box, box, vfd.F32)
+    a = np.random.default_rng(q).standard_normal(box).astype(np.float32)
+    spec = torch.empty(box[:2] + (q + 1,), dtype=torch.complex64, device="cuda")
+    back = torch.empty(box, device="cuda")
+    plan.r2c(torch.from_numpy(a).cuda(), spec)
+    got = spec.cpu().numpy()
+    plan.c2r(spec, back)
+    ref = np.fft.rfftn(a.astype(np.float64))
+    tol = 2.0 ** -23 * np.log2(a.size)
+    assert np.abs(got - ref).max() <= tol * np.abs(ref).max()
+    assert np.abs(back.cpu().numpy().astype(np.float64) / a.size - a).max() <= 2 * tol * np.abs(a).max()

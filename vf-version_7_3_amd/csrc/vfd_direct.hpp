@@ -325,7 +325,7 @@ template <int A> __device__ __forceinline__ float4 dir_ld4(rsrc_t r, unsigned of
 
 // x and y windows of one strip: TX columns from x0, rows [y0, y1) of plane z.
 // Bound by vector instructions, 0.96 of its cycles: 8 fields 1024x512x128 (R 6 - 19)
-// in 0.99 ms, 4.4 TB/s (1.08 ms one output at a time).
+// in 1.02 ms, 4.2 TB/s (1.12 ms one output at a time).
 template <int TX, int RB>
 __device__ __forceinline__ void dir_xy_strip(float* lds, const DirRecord* rec, rsrc_t rin, rsrc_t rw, const DirDims& d,
                                              int z, int x0, int y0, int y1) {
